@@ -10,14 +10,16 @@
 // per-wave partials through LDS. The row is read from HBM exactly once and
 // the output written once.
 //
-// Streaming path (widths that are not a multiple of the 16-byte vector, or
-// too wide for registers): one 256-thread block per row, scalar accesses,
-// the row re-read for every pass.
+// Rows of other widths and alignments: k_rowany.hip. Streaming path (what
+// that does not take: rows of less than one vector, and rows of more than
+// 4096 vectors under stream capture): one 256-thread block per row, scalar
+// accesses, the row re-read for every pass.
 //
 // Accumulation is f32; the order is per-lane sequential then a tree, which
 // differs from the reference's single sequential sum only by rounding.
 #include "kern_common.hpp"
 #include "kernels.hpp"
+#include "row_any.hpp"
 
 namespace icsdk {
 namespace {
@@ -587,6 +589,10 @@ inline bool pick_row_shape(size_t width, size_t elem, bool aligned, RowShape *sh
     return false;
 }
 
+// Rows that are not taken by the register kernels here: not whole aligned
+// vectors, too long, or so narrow that several share a wave (row_any).
+inline bool narrow(size_t width, size_t elem) { return width * elem <= 16 * row_any::kNarrowVectors; }
+
 inline dim3 row_grid(size_t rows, int wpr) {
     const size_t per_block = wpr == 1 ? kBlock / kWave : 1;
     return dim3((unsigned)((rows + per_block - 1) / per_block));
@@ -621,7 +627,7 @@ hipError_t launch_rms(const S *x, const S *residual, S *sum_out, const S *w, S *
     // the two shapes tie. (The causal softmax keeps one wave per row: four
     // cost it 30%.)
     const int wpr_first = rows >= 8192 && width * sizeof(S) >= 16u * 4 * kWave ? 4 : 1;
-    if (pick_row_shape(width, sizeof(S), aligned, &shape, wpr_first)) {
+    if (!narrow(width, sizeof(S)) && pick_row_shape(width, sizeof(S), aligned, &shape, wpr_first)) {
         const bool exact = width / (16 / sizeof(S)) == (size_t)shape.nv * shape.wpr * kWave;
 #define ICSDK_RMS(NV, WPR)                                                                 \
     do {                                                                                   \
@@ -637,6 +643,8 @@ hipError_t launch_rms(const S *x, const S *residual, S *sum_out, const S *w, S *
         ICSDK_ROW_DISPATCH(shape, ICSDK_RMS);
 #undef ICSDK_RMS
     } else {
+        const hipError_t e = row_any::rms_norm<S>(x, residual, sum_out, w, y, rows, width, eps, s);
+        if (e != hipErrorNotSupported) return e;
         // one block per row: the grid's x dimension holds at most 2^32 - 1
         if (rows > 0xffffffffu) return hipErrorInvalidValue;
         hipLaunchKernelGGL((rms_norm_stream_kernel<S, kResidual>), dim3((unsigned)rows),
@@ -651,7 +659,7 @@ hipError_t launch_layer(const S *x, const S *scale, const S *bias, S *y, size_t 
     if (rows == 0) return hipSuccess;
     RowShape shape;
     const bool aligned = aligned16(x) && aligned16(scale) && aligned16(bias) && aligned16(y);
-    if (pick_row_shape(width, sizeof(S), aligned, &shape)) {
+    if (!narrow(width, sizeof(S)) && pick_row_shape(width, sizeof(S), aligned, &shape)) {
         const bool exact = width / (16 / sizeof(S)) == (size_t)shape.nv * shape.wpr * kWave;
         const int affine = (scale ? 1 : 0) + (bias ? 2 : 0);
 #define ICSDK_LN_GO(NV, WPR, EX, SC, BI)                                                    \
@@ -676,6 +684,8 @@ hipError_t launch_layer(const S *x, const S *scale, const S *bias, S *y, size_t 
 #undef ICSDK_LN_AFF
 #undef ICSDK_LN_GO
     } else {
+        const hipError_t e = row_any::layer_norm<S>(x, scale, bias, y, rows, width, eps, s);
+        if (e != hipErrorNotSupported) return e;
         // one block per row: the grid's x dimension holds at most 2^32 - 1
         if (rows > 0xffffffffu) return hipErrorInvalidValue;
         hipLaunchKernelGGL((layer_norm_stream_kernel<S>), dim3((unsigned)rows), dim3(kBlock),
@@ -691,7 +701,8 @@ hipError_t launch_softmax(const S *x, S *y, size_t rows, size_t width, size_t q_
     const size_t offset = q_len && width > q_len ? width - q_len : 0;
     RowShape shape;
     const bool aligned = aligned16(x) && aligned16(y);
-    if (q_len <= 0xffffffffu && pick_row_shape(width, sizeof(S), aligned, &shape)) {
+    if (q_len <= 0xffffffffu && !narrow(width, sizeof(S)) &&
+        pick_row_shape(width, sizeof(S), aligned, &shape)) {
         const FastDiv qd = make_fast_div(q_len ? (uint32_t)q_len : 1u);
 #define ICSDK_SM(NV, WPR)                                                                  \
     hipLaunchKernelGGL((softmax_kernel<S, NV, WPR>), row_grid(rows, WPR), dim3(kBlock), 0, \
@@ -700,6 +711,8 @@ hipError_t launch_softmax(const S *x, S *y, size_t rows, size_t width, size_t q_
         ICSDK_ROW_DISPATCH(shape, ICSDK_SM);
 #undef ICSDK_SM
     } else {
+        const hipError_t e = row_any::softmax<S>(x, y, rows, width, q_len, offset, s);
+        if (e != hipErrorNotSupported) return e;
         // one block per row: the grid's x dimension holds at most 2^32 - 1
         if (rows > 0xffffffffu) return hipErrorInvalidValue;
         hipLaunchKernelGGL((softmax_stream_kernel<S>), dim3((unsigned)rows), dim3(kBlock), 0,
@@ -713,13 +726,15 @@ hipError_t launch_row_reduce(const S *x, float *y, size_t rows, size_t width,
                              hipStream_t s) {
     if (rows == 0) return hipSuccess;
     RowShape shape;
-    if (pick_row_shape(width, sizeof(S), aligned16(x), &shape)) {
+    if (!narrow(width, sizeof(S)) && pick_row_shape(width, sizeof(S), aligned16(x), &shape)) {
 #define ICSDK_RR(NV, WPR)                                                                  \
     hipLaunchKernelGGL((row_reduce_kernel<S, NV, WPR, kMax>), row_grid(rows, WPR),         \
                        dim3(kBlock), 0, s, x, y, rows, (uint32_t)width)
         ICSDK_ROW_DISPATCH(shape, ICSDK_RR);
 #undef ICSDK_RR
     } else {
+        const hipError_t e = row_any::reduce<S, kMax>(x, y, rows, width, s);
+        if (e != hipErrorNotSupported) return e;
         // one block per row: the grid's x dimension holds at most 2^32 - 1
         if (rows > 0xffffffffu) return hipErrorInvalidValue;
         hipLaunchKernelGGL((row_reduce_stream_kernel<S, kMax>), dim3((unsigned)rows),
