@@ -19,10 +19,12 @@
 //             this beats staging the same permutation through LDS tiles at
 //             every run length from 16 to 256 bytes;
 //   tile    - x's contiguous dimension is another view dimension p (a
-//             transpose of p with the innermost dimension): 64x64 tiles are
-//             read along p, staged through LDS (padded against bank
+//             transpose of p with the innermost dimension): tiles are read
+//             along p, staged through LDS (swizzled or padded against bank
 //             conflicts) and written along the innermost dimension, so both
-//             HBM streams stay coalesced;
+//             HBM streams stay coalesced: 64x64 tiles in 16-byte vectors of
+//             any alignment where both dimensions have 64 elements, else
+//             tiles of about 4096 elements shaped to the smaller one;
 //   scalar  - anything else: one element per lane.
 #include "kern_common.hpp"
 #include "kernels.hpp"
@@ -303,9 +305,11 @@ __global__ __launch_bounds__(kBlock) void view_scalar_kernel(const S *__restrict
 // ---- LDS-tiled transpose path ------------------------------------------------
 
 // Output dims are viewed as [outer..., P, inner..., L] where dimension p has
-// x stride 1 and L is the last view dimension. A block moves one 64x64 tile
-// of (p, last) for one combination of the remaining indices ("batch").
+// x stride 1 and L is the last view dimension. A block moves one tile of (p,
+// last) for one combination of the remaining indices ("batch").
 constexpr int kTile = 64;
+constexpr uint32_t kTileElems = 4096;      // elements per block of the adaptive tiles, or
+constexpr uint32_t kTileElemsSmall = 1024; // for small views
 
 struct TilePlan {
     int rank;
@@ -318,85 +322,130 @@ struct TilePlan {
     uint64_t x_offset;
     uint64_t batches;               // product of the dims other than p and last
     uint32_t tiles_p, tiles_l;
+    FastDiv tile_p, tile_l;         // the adaptive tile's extents
 };
 
-template <typename S>
+// The product as the f32 value it is. (The compiler otherwise folds a f32
+// multiply and its conversion to f16 into v_fma_mixlo_f16, which rounds once:
+// another result at ties.)
+template <typename S> __device__ inline float rounded_f32(float v) {
+    if constexpr (sizeof(S) == 2) asm("" : "+v"(v));
+    return v;
+}
+
+// Where a batch starts in each operand.
+struct BatchBase {
+    int64_t x;
+    uint64_t a, m, y;
+    __device__ BatchBase(const TilePlan &plan, uint64_t batch)
+        : x((int64_t)plan.x_offset), a(0), m(0), y(0) {
+        if (batch == 0) return;   // block-uniform
+        for (int d = plan.rank - 2; d >= 0; --d) {
+            if (d == plan.p) continue;
+            const uint64_t idx = batch % plan.shape[d];
+            batch /= plan.shape[d];
+            x += (int64_t)idx * plan.x_stride[d];
+            a += idx * plan.a_stride[d];
+            m += idx * plan.m_stride[d];
+            y += idx * plan.y_stride[d];
+        }
+    }
+};
+
+// Tiles of tile_p x tile_l elements, about kTileElems in all: with a short p
+// (the channels of an image stored channel-last) or a short last dimension
+// the other one is long, so a block still moves 4096 elements and both its
+// reads and its writes run along memory. One element per lane and access, 16
+// of each lane in flight; reads past the tile are clamped onto its first
+// element and not stored. LDS rows [l], pitch odd: conflict-free both ways.
+// NHWC [8, 512, 512, 3] f32 to NCHW 117 -> 11.7 us, with both operands 122 ->
+// 16.4 (64 x 64 tiles, 61 of 64 columns empty, before).
+template <typename S, uint32_t kElems, bool kA, bool kM>
 __global__ __launch_bounds__(kBlock) void view_tile_kernel(const S *__restrict__ x,
                                                            const S *__restrict__ addend,
                                                            const S *__restrict__ mult,
                                                            S *__restrict__ y, TilePlan plan) {
-    __shared__ float tile[kTile][kTile + 1];
+    __shared__ S tile[kElems / 2 * 3];   // tile_l * pitch (the host checks)
+    constexpr int kPer = kElems / kBlock;
     const int last = plan.rank - 1;
     const uint64_t block = blockIdx.x;
     const uint32_t tl = (uint32_t)(block % plan.tiles_l);
     const uint32_t tp = (uint32_t)((block / plan.tiles_l) % plan.tiles_p);
-    uint64_t batch = block / ((uint64_t)plan.tiles_l * plan.tiles_p);
-    // base offsets from the batch index (dims other than p and last)
-    int64_t xb = (int64_t)plan.x_offset;
-    uint64_t ab = 0, mb = 0, yb = 0;
-    for (int d = last - 1; d >= 0; --d) {
-        if (d == plan.p) continue;
-        const uint64_t idx = batch % plan.shape[d];
-        batch /= plan.shape[d];
-        xb += (int64_t)idx * plan.x_stride[d];
-        ab += idx * plan.a_stride[d];
-        mb += idx * plan.m_stride[d];
-        yb += idx * plan.y_stride[d];
+    const BatchBase base(plan, block / ((uint64_t)plan.tiles_l * plan.tiles_p));
+    const uint32_t ep = plan.tile_p.divisor, el = plan.tile_l.divisor, pitch = ep | 1u;
+    const uint64_t p0 = (uint64_t)tp * ep, l0 = (uint64_t)tl * el;
+    const uint32_t np = (uint32_t)min((uint64_t)ep, plan.shape[plan.p] - p0);
+    const uint32_t nl = (uint32_t)min((uint64_t)el, plan.shape[last] - l0);
+    // read: consecutive lanes walk p (contiguous in x), then l
+    const int64_t xl = plan.x_stride[last];
+    const S *xt = x + base.x + (int64_t)p0 + (int64_t)l0 * xl;
+    S v[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const uint32_t t = threadIdx.x + k * kBlock, l = fast_div(t, plan.tile_p), p = t - l * ep;
+        v[k] = xt[p < np && l < nl ? (int64_t)l * xl + p : 0];
     }
-    const uint64_t p0 = (uint64_t)tp * kTile, l0 = (uint64_t)tl * kTile;
-    const uint64_t np = plan.shape[plan.p], nl = plan.shape[last];
-    // read: consecutive threads walk p (contiguous in x)
-    const uint32_t tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;
-    for (uint32_t r = ty; r < kTile; r += kBlock / kTile) {
-        const uint64_t pi = p0 + tx, li = l0 + r;
-        if (pi < np && li < nl)
-            tile[r][tx] = Elem<S>::load(x[xb + (int64_t)pi * plan.x_stride[plan.p] +
-                                          (int64_t)li * plan.x_stride[last]]);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const uint32_t t = threadIdx.x + k * kBlock, l = fast_div(t, plan.tile_p), p = t - l * ep;
+        if (l < el) tile[l * pitch + p] = v[k];
     }
     __syncthreads();
-    // write: consecutive threads walk the last dim (contiguous in y)
-    for (uint32_t r = ty; r < kTile; r += kBlock / kTile) {
-        const uint64_t pi = p0 + r, li = l0 + tx;
-        if (pi < np && li < nl) {
-            float v = tile[tx][r];
-            if (addend) v = v + Elem<S>::load(addend[ab + pi * plan.a_stride[plan.p] +
-                                                      li * plan.a_stride[last]]);
-            if (mult) v = v * Elem<S>::load(mult[mb + pi * plan.m_stride[plan.p] +
-                                                  li * plan.m_stride[last]]);
-            y[yb + pi * plan.y_stride[plan.p] + li] = Elem<S>::store(v);
-        }
+    // write: consecutive lanes walk the last dim (contiguous in y), then p
+    const uint64_t ap = plan.a_stride[plan.p], al = plan.a_stride[last];
+    const uint64_t mp = plan.m_stride[plan.p], ml = plan.m_stride[last], yp = plan.y_stride[plan.p];
+    const S *at = kA ? addend + base.a + p0 * ap + l0 * al : nullptr;
+    const S *mt = kM ? mult + base.m + p0 * mp + l0 * ml : nullptr;
+    S *yt = y + base.y + p0 * yp + l0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const uint32_t t = threadIdx.x + k * kBlock, p = fast_div(t, plan.tile_l), l = t - p * el;
+        const bool in = p < np && l < nl;
+        float r = Elem<S>::load(tile[in ? l * pitch + p : 0]);
+        if constexpr (kA) r = r + Elem<S>::load(at[in ? p * ap + l * al : 0]);
+        if constexpr (kM) r = rounded_f32<S>(r * Elem<S>::load(mt[in ? p * mp + l * ml : 0]));
+        if (in) yt[p * yp + l] = Elem<S>::store(r);
     }
 }
 
-// Transposes without operands in whole 16-byte vectors of E elements (8 for
-// f16, 4 for f32; the tile's dims and every row start a multiple of E
-// elements and 16-byte aligned; the launcher checks): a tile's 64 x rows (64
-// elements along p, contiguous in x) are read as 64 / E vectors each into LDS
-// rows [l], vector c of row l at slot c ^ (l / E); each output row (64
-// elements along the last dim, contiguous in y) is gathered from one LDS
+// 64 x 64 tiles in 16-byte vectors of E elements (8 for f16, 4 for f32), for
+// views whose p and last dimensions have at least 64 elements: a tile's 64 x
+// rows (64 elements along p, contiguous in x) are read as 64 / E vectors each
+// into LDS rows [l], vector c of row l at slot c ^ (l / E); each output row
+// (64 elements along the last dim, contiguous in y) is gathered from one LDS
 // column, E reads per vector, and written as 64 / E vectors. With the slot
 // swizzle the 64 lanes of a gather read distinct banks (f16: 32, lanes 2m
-// and 2m + 1 sharing a dword; f32: 64). A block takes
-// kVecTiles tiles along the last dim, all of a lane's loads issued first
-// ([4096, 4096]: one tile per block 15.0 us, two 13.1, four 12.7-12.8). The
-// scalar kernel below moves one element per lane per access.
+// and 2m + 1 sharing a dword; f32: 64). A last tile that would reach past the
+// end starts 64 elements before it instead and writes the overlap with the
+// same values, so no access needs a bounds test; vectors are loaded and
+// stored at any element alignment. A block takes kTiles tiles along the last dim: two for f16 where
+// that still leaves 1024 blocks, else one (f16 with an addend, one / two /
+// four tiles: [3000, 3000] 13.7 / 10.0 / 11.3 us, [8192, 8192] 48.9 / 47.0 /
+// 47.9, [4096, 4096] 13.4 / 15.0 / 16.4). kGuarded: the form for f16 whole
+// aligned vectors without operands: bounds tests instead of the overlap,
+// four tiles, each load waited for before the next, which is the faster one
+// there ([4096, 4000] 11.6 us against 12.7-12.8, [64, 512, 512] 12.4 against
+// 13.2-15.6). Operands enter as a vector along the last dim or as one element per
+// output row (OperandKind), loaded before the barrier. Against the
+// one-element-per-lane tiles: f16 [4097, 4095] 30.0 -> 21.4 us, [4096,
+// 4096] with both operands 41.0 -> 15.1, f32 39.6 -> 26.0.
 //
 // Everything a wave needs before its first load arrives as a plain scalar
 // argument (preloaded in SGPRs; the tile grid split by multiply-high
-// divisions); the plan is read only by blocks past the first batch.
-// 64 x 64 tiles per block along the last dim: 4 for 2-byte elements (32 KB
-// of LDS), 1 for f32 (16 KB; f32 [4096, 4096]: 29.7 us with 2, 27.7 with 1)
-template <typename S> constexpr uint32_t kVecTiles = sizeof(S) == 2 ? 4 : 1;
-template <typename S>
+// divisions); the plan is read only by blocks past the first batch and for
+// the operands.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+template <typename S, uint32_t kTiles, int kA, int kM, bool kGuarded = false>
 __global__ __launch_bounds__(kBlock) void view_tile_vec_kernel(
     const S *__restrict__ x, S *__restrict__ y, uint32_t tiles_l, uint32_t tl_mul,
     uint32_t tl_shift, uint32_t tiles_p, uint32_t tp_mul, uint32_t tp_shift, uint32_t np,
-    uint32_t nl, uint32_t xs_last, uint32_t x_offset, uint32_t ys, TilePlan plan) {
+    uint32_t nl, uint32_t xs_last, uint32_t x_offset, uint32_t ys, const S *__restrict__ addend,
+    const S *__restrict__ mult, TilePlan plan) {
     static_assert(sizeof(S) == 2 || sizeof(S) == 4, "2- or 4-byte elements");
     constexpr uint32_t E = Vec16<S>::N;              // elements per 16-byte vector
     constexpr uint32_t kSlots = kTile / E;           // vectors per 64-element row
     constexpr uint32_t kRowsPerPass = kBlock / kSlots;
-    constexpr uint32_t kTiles = kVecTiles<S>;
+    constexpr uint32_t kPasses = kTile / kRowsPerPass;
     using U = std::conditional_t<sizeof(S) == 2, uint16_t, uint32_t>;
     __shared__ u32x4 tile[kTiles][kTile][kSlots];
     const uint32_t block = blockIdx.x;
@@ -405,54 +454,89 @@ __global__ __launch_bounds__(kBlock) void view_tile_vec_kernel(
     uint32_t batch = fast_div(rest, FastDiv{tiles_p, tp_mul, tp_shift});
     const uint32_t tp = rest - batch * tiles_p;
     int64_t xb = (int64_t)x_offset;
-    uint64_t yb = 0;
+    uint64_t yb = 0, ab = 0, mb = 0;
     if (batch != 0) {   // block-uniform; batch 0 has every batch index 0
-        const int last = plan.rank - 1;
-        uint64_t b = batch;
-        for (int d = last - 1; d >= 0; --d) {
-            if (d == plan.p) continue;
-            const uint64_t idx = b % plan.shape[d];
-            b /= plan.shape[d];
-            xb += (int64_t)idx * plan.x_stride[d];
-            yb += idx * plan.y_stride[d];
-        }
+        const BatchBase base(plan, batch);
+        xb = base.x;
+        yb = base.y;
+        ab = base.a;
+        mb = base.m;
     }
-    const uint32_t p0 = tp * kTile, l0 = tl * (kTiles * kTile);
-    const uint32_t c = threadIdx.x % kSlots;
+    const uint32_t p0 = kGuarded ? tp * kTile : min(tp * kTile, np - kTile);
+    const uint32_t c = threadIdx.x % kSlots, r0 = threadIdx.x / kSlots;
+    // the first index of tile tt along the last dim; tiles past the end repeat
+    // the last one (and store nothing)
+    auto first_l = [&](uint32_t tt) {
+        const uint32_t l = (tl * kTiles + tt) * kTile;
+        return kGuarded ? l : min(l, nl - kTile);
+    };
 #pragma unroll
     for (uint32_t tt = 0; tt < kTiles; ++tt)
 #pragma unroll
-    for (uint32_t pass = 0; pass < kTile / kRowsPerPass; ++pass) {
-        const uint32_t l = threadIdx.x / kSlots + kRowsPerPass * pass;
-        const uint32_t li = l0 + kTile * tt + l, pi = p0 + E * c;
-        u32x4 v = u32x4{0u, 0u, 0u, 0u};
-        if (li < nl && pi < np)
-            v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(
-                x + xb + (int64_t)li * xs_last + pi));
+    for (uint32_t pass = 0; pass < kPasses; ++pass) {
+        const uint32_t l = r0 + kRowsPerPass * pass;
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (!kGuarded || (first_l(tt) + l < nl && p0 + E * c < np))
+            v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any *>(
+                x + xb + (int64_t)(first_l(tt) + l) * xs_last + p0 + E * c));
         tile[tt][l][c ^ (l / E % kSlots)] = v;
+    }
+    // operands of this lane's output vectors
+    Vec16<S> av[kA == kVector ? kTiles * kPasses : 1], mv[kM == kVector ? kTiles * kPasses : 1];
+    float as[kA == kScalar ? kPasses : 1], ms[kM == kScalar ? kPasses : 1];
+    if constexpr (kA != kNone || kM != kNone) {
+        const uint64_t ap = plan.a_stride[plan.p], mp = plan.m_stride[plan.p];
+#pragma unroll
+        for (uint32_t pass = 0; pass < kPasses; ++pass) {
+            const uint64_t pi = p0 + r0 + kRowsPerPass * pass;
+            if constexpr (kA == kScalar) as[pass] = Elem<S>::load(addend[ab + pi * ap]);
+            if constexpr (kM == kScalar) ms[pass] = Elem<S>::load(mult[mb + pi * mp]);
+#pragma unroll
+            for (uint32_t tt = 0; tt < kTiles; ++tt) {
+                const uint32_t li = first_l(tt) + E * c;
+                if constexpr (kA == kVector)
+                    av[tt * kPasses + pass] = __builtin_bit_cast(
+                        Vec16<S>, (u32x4)*reinterpret_cast<const u32x4_any *>(addend + ab + pi * ap + li));
+                if constexpr (kM == kVector)
+                    mv[tt * kPasses + pass] = __builtin_bit_cast(
+                        Vec16<S>, (u32x4)*reinterpret_cast<const u32x4_any *>(mult + mb + pi * mp + li));
+            }
+        }
     }
     __syncthreads();
 #pragma unroll
     for (uint32_t tt = 0; tt < kTiles; ++tt)
 #pragma unroll
-    for (uint32_t pass = 0; pass < kTile / kRowsPerPass; ++pass) {
-        const uint32_t pr = threadIdx.x / kSlots + kRowsPerPass * pass;
-        const uint32_t pi = p0 + pr, li = l0 + kTile * tt + E * c;
-        if (pi < np && li < nl) {
-            // element (l = E c + k, p = pr): row l, slot (pr / E) ^ c, element pr % E
-            uint32_t h[E];
+    for (uint32_t pass = 0; pass < kPasses; ++pass) {
+        const uint32_t pr = r0 + kRowsPerPass * pass;
+        if (kGuarded && (p0 + pr >= np || first_l(tt) + E * c >= nl)) continue;
+        // element (l = E c + k, p = pr): row l, slot (pr / E) ^ c, element pr % E
+        uint32_t h[E];
+#pragma unroll
+        for (uint32_t k = 0; k < E; ++k) {
+            const U *row = reinterpret_cast<const U *>(&tile[tt][E * c + k][0]);
+            h[k] = row[(((pr / E) ^ c) * E) + pr % E];
+        }
+        u32x4 o;
+        if constexpr (sizeof(S) == 2)
+            o = u32x4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+        else
+            o = u32x4{h[0], h[1], h[2], h[3]};
+        if constexpr (kA != kNone || kM != kNone) {
+            Vec16<S> ov = __builtin_bit_cast(Vec16<S>, o);
 #pragma unroll
             for (uint32_t k = 0; k < E; ++k) {
-                const U *row = reinterpret_cast<const U *>(&tile[tt][E * c + k][0]);
-                h[k] = row[(((pr / E) ^ c) * E) + pr % E];
+                float r = Elem<S>::load(ov.v[k]);
+                if constexpr (kA == kVector) r = r + Elem<S>::load(av[tt * kPasses + pass].v[k]);
+                if constexpr (kA == kScalar) r = r + as[pass];
+                if constexpr (kM == kVector) r = rounded_f32<S>(r * Elem<S>::load(mv[tt * kPasses + pass].v[k]));
+                if constexpr (kM == kScalar) r = rounded_f32<S>(r * ms[pass]);
+                ov.v[k] = Elem<S>::store(r);
             }
-            u32x4 o;
-            if constexpr (sizeof(S) == 2)
-                o = u32x4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
-            else
-                o = u32x4{h[0], h[1], h[2], h[3]};
-            *reinterpret_cast<u32x4 *>(y + yb + (uint64_t)pi * ys + li) = o;
+            o = __builtin_bit_cast(u32x4, ov);
         }
+        if (kTiles == 1 || kGuarded || (tl * kTiles + tt) * kTile < nl)
+            *reinterpret_cast<u32x4_any *>(y + yb + (uint64_t)(p0 + pr) * ys + first_l(tt) + E * c) = o;
     }
 }
 
@@ -612,41 +696,82 @@ hipError_t launch_view(const S *x, const k::ViewArgs &v, const S *addend,
         }
         plan.x_offset = v.offset;
         plan.batches = n / (c.shape[p] * c.shape[last]);
-        plan.tiles_p = (uint32_t)((c.shape[p] + kTile - 1) / kTile);
-        plan.tiles_l = (uint32_t)((c.shape[last] + kTile - 1) / kTile);
-        const uint64_t blocks = plan.batches * plan.tiles_p * plan.tiles_l;
-        if (blocks < (uint64_t{1} << 31)) {
-            {
-                // whole 16-byte vectors: p and last a multiple of E elements,
-                // every x row and batch offset too, both tensors 16-byte aligned
-                // (the scalar arguments hold dims, the x row stride, the
-                // offset and the output row stride in 32 bits)
-                const uint64_t lim = 0xffffffffull;
-                constexpr uint64_t E = Vec16<S>::N;
-                bool vec = addend == nullptr && mult == nullptr && c.shape[p] % E == 0 &&
-                           c.shape[last] % E == 0 && v.offset % E == 0 &&
-                           ((uintptr_t)x & 15u) == 0 && ((uintptr_t)y & 15u) == 0 &&
-                           c.shape[p] + kTile <= lim && c.shape[last] + kTile <= lim &&
-                           c.x_stride[last] > 0 && (uint64_t)c.x_stride[last] <= lim &&
-                           v.offset <= lim && plan.y_stride[p] <= lim;
-                for (int d = 0; d <= last; ++d)
-                    if (d != p && c.x_stride[d] % (int64_t)E != 0) vec = false;
-                if (vec) {
-                    const uint32_t pairs_l = (plan.tiles_l + kVecTiles<S> - 1) / kVecTiles<S>;
-                    const uint64_t vblocks = plan.batches * plan.tiles_p * pairs_l;
-                    const FastDiv dl = make_fast_div(pairs_l), dp = make_fast_div(plan.tiles_p);
-                    hipLaunchKernelGGL((view_tile_vec_kernel<S>), dim3((unsigned)vblocks),
-                                       dim3(kBlock), 0, s, x, y, pairs_l, dl.multiplier,
-                                       dl.shift, plan.tiles_p, dp.multiplier, dp.shift,
-                                       (uint32_t)c.shape[p], (uint32_t)c.shape[last],
-                                       (uint32_t)c.x_stride[last], (uint32_t)v.offset,
-                                       (uint32_t)plan.y_stride[p], plan);
+        const uint64_t np = c.shape[p], nl = c.shape[last], lim = 0xffffffffull;
+        const int ka = !addend ? kNone : c.a_stride[last] != 0 ? kVector : kScalar;
+        const int km = !mult ? kNone : c.m_stride[last] != 0 ? kVector : kScalar;
+        // 64 x 64 tiles of vectors: both dims of at least 64 elements (the
+        // scalar arguments hold dims, the x row stride, the offset and the
+        // output row stride in 32 bits; the operands' rows run along last)
+        if (np >= kTile && nl >= kTile && np + kTile <= lim && nl + 4 * kTile <= lim &&
+            c.x_stride[last] > 0 && (uint64_t)c.x_stride[last] <= lim && v.offset <= lim &&
+            plan.y_stride[p] <= lim && c.a_stride[last] <= 1 && c.m_stride[last] <= 1) {
+            plan.tiles_p = (uint32_t)((np + kTile - 1) / kTile);
+            const uint64_t all_tiles = plan.batches * plan.tiles_p * ((nl + kTile - 1) / kTile);
+            // whole aligned vectors in every x row, batch offset and output row
+            constexpr uint64_t E = Vec16<S>::N;
+            bool guarded = sizeof(S) == 2 && !addend && !mult && np % E == 0 && nl % E == 0 &&
+                           v.offset % E == 0 && aligned16(x) && aligned16(y);
+            for (int d = 0; d <= last; ++d)
+                if (d != p && c.x_stride[d] % (int64_t)E != 0) guarded = false;
+            const uint32_t per = guarded ? 4 : sizeof(S) == 2 && all_tiles >= 2048 && nl > kTile ? 2 : 1;
+            const uint32_t spans_l = (uint32_t)((nl + per * kTile - 1) / (per * kTile));
+            const uint64_t vblocks = plan.batches * plan.tiles_p * spans_l;
+            if (vblocks < (uint64_t{1} << 24)) {
+                const FastDiv dl = make_fast_div(spans_l), dp = make_fast_div(plan.tiles_p);
+                auto go = [&](auto kernel) {
+                    hipLaunchKernelGGL(kernel, dim3((unsigned)vblocks), dim3(kBlock), 0, s, x, y, spans_l,
+                                       dl.multiplier, dl.shift, plan.tiles_p, dp.multiplier, dp.shift,
+                                       (uint32_t)np, (uint32_t)nl, (uint32_t)c.x_stride[last],
+                                       (uint32_t)v.offset, (uint32_t)plan.y_stride[p], addend, mult, plan);
                     return hipGetLastError();
+                };
+#define ICSDK_TILE_VEC(A, M)                                                                     \
+    do {                                                                                         \
+        if constexpr (sizeof(S) == 2)                                                            \
+            if (per == 2) return go(view_tile_vec_kernel<S, 2, A, M>);                           \
+        return go(view_tile_vec_kernel<S, 1, A, M>);                                             \
+    } while (0)
+                if constexpr (sizeof(S) == 2)
+                    if (guarded) return go(view_tile_vec_kernel<S, 4, kNone, kNone, true>);
+                switch (ka * 3 + km) {
+                    case 0: ICSDK_TILE_VEC(kNone, kNone);
+                    case 1: ICSDK_TILE_VEC(kNone, kVector);
+                    case 2: ICSDK_TILE_VEC(kNone, kScalar);
+                    case 3: ICSDK_TILE_VEC(kVector, kNone);
+                    case 4: ICSDK_TILE_VEC(kVector, kVector);
+                    case 5: ICSDK_TILE_VEC(kVector, kScalar);
+                    case 6: ICSDK_TILE_VEC(kScalar, kNone);
+                    case 7: ICSDK_TILE_VEC(kScalar, kVector);
+                    default: ICSDK_TILE_VEC(kScalar, kScalar);
                 }
+#undef ICSDK_TILE_VEC
             }
-            hipLaunchKernelGGL((view_tile_kernel<S>), dim3((unsigned)blocks), dim3(kBlock), 0,
-                               s, x, addend, mult, y, plan);
-            return hipGetLastError();
+        }
+        // adaptive tiles: the shorter dim whole up to 64 (32 for small
+        // tiles), the other one as long as fits the tile; views of fewer than
+        // 1024 large tiles take small ones (more, shorter blocks)
+        const bool small = n <= 1024ull * kTileElems;
+        const uint64_t elems = small ? kTileElemsSmall : kTileElems, side = small ? 32 : 64;
+        uint64_t ep = std::min(np, side), el = std::min(nl, side);
+        if (np <= nl) el = std::min(nl, std::max<uint64_t>(elems / ep / side, 1) * side);
+        else ep = std::min(np, std::max<uint64_t>(elems / el / side, 1) * side);
+        plan.tile_p = make_fast_div((uint32_t)ep);
+        plan.tile_l = make_fast_div((uint32_t)el);
+        plan.tiles_p = (uint32_t)((np + ep - 1) / ep);
+        plan.tiles_l = (uint32_t)((nl + el - 1) / el);
+        const uint64_t blocks = plan.batches * plan.tiles_p * plan.tiles_l;
+        if (blocks < (uint64_t{1} << 24) && ep * el <= elems && (ep | 1u) * el <= elems / 2 * 3) {
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, x, addend, mult, y, plan);
+                return hipGetLastError();
+            };
+#define ICSDK_TILE(A, M)                                                                           \
+    return small ? go(view_tile_kernel<S, kTileElemsSmall, A, M>) : go(view_tile_kernel<S, kTileElems, A, M>)
+            if (addend && mult) ICSDK_TILE(true, true);
+            if (addend) ICSDK_TILE(true, false);
+            if (mult) ICSDK_TILE(false, true);
+            ICSDK_TILE(false, false);
+#undef ICSDK_TILE
         }
     }
 

@@ -1,0 +1,66 @@
+"""Transposing views at the edges of their tiles, with and without operands,
+against numpy (one or two IEEE operations in f32, rounded once: exact)."""
+import numpy as np
+import pytest
+
+from inference_c_amd.sdk import TensorView
+
+pytestmark = pytest.mark.gpu
+
+# stored shape, axis order of the view
+CASES = [
+    ((64, 64), (1, 0)), ((65, 64), (1, 0)), ((63, 64), (1, 0)), ((67, 129), (1, 0)),
+    ((513, 191), (1, 0)), ((300, 66), (1, 0)), ((3, 70, 200), (0, 2, 1)), ((5, 1000, 65), (0, 2, 1)),
+    ((40, 900, 1000), (0, 2, 1)),            # four tiles per block (f16)
+    ((2, 31, 37, 3), (0, 3, 1, 2)), ((3, 64, 64, 4), (0, 3, 1, 2)), ((1, 50, 41, 2), (0, 3, 1, 2)),
+    ((2, 3, 31, 37), (0, 2, 3, 1)), ((1, 16, 65, 9), (0, 2, 3, 1)), ((2, 63, 20, 70), (0, 2, 3, 1)),
+    ((33, 17, 65), (2, 0, 1)), ((9, 8, 7, 6), (3, 2, 1, 0)), ((70, 5, 66), (2, 1, 0)),
+    ((2, 5000), (1, 0)), ((5000, 2), (1, 0)), ((1, 3), (1, 0)),
+]
+
+
+def broadcast(kind, shape):
+    if kind is None:
+        return None
+    keep = {"last": {len(shape) - 1}, "first": {0}, "second": {1}, "full": set(range(len(shape))),
+            "one": set()}[kind]
+    return tuple(n if i in keep else 1 for i, n in enumerate(shape))
+
+
+@pytest.mark.parametrize("shape,order", CASES)
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("add,mul", [(None, None), ("last", None), (None, "last"), ("second", "second"),
+                                     ("full", "one"), ("one", "full"), ("last", "first")])
+def test_transposing_view(sdk, orc, shape, order, dtype, add, mul):
+    np_type = np.float16 if dtype == "f16" else np.float32
+    x = orc.normal(shape, 91, 0, 0.0, 1.0, dtype)
+    out = tuple(shape[i] for i in order)
+    a_shape, m_shape = broadcast(add, out), broadcast(mul, out)
+    a = None if add is None else orc.normal(a_shape, 91, 1, 0.0, 1.0, dtype)
+    m = None if mul is None else orc.normal(m_shape, 91, 2, 1.0, 1.0, dtype)
+    strides = [int(np.prod(shape[i + 1:])) for i in range(len(shape))]
+    view = TensorView.make(out, [strides[i] for i in order])
+    ty = sdk.tensor(dtype, out)
+    sdk.call(f"tensor_view_add_mul_{dtype}", sdk.from_numpy(x), view,
+             None if a is None else sdk.from_numpy(a), None if m is None else sdk.from_numpy(m), ty)
+    want = np.ascontiguousarray(x.transpose(order)).astype(np.float32)
+    if a is not None:
+        want = want + a.astype(np.float32)
+    if m is not None:
+        want = want * m.astype(np.float32)
+    assert np.array_equal(ty.download(), want.astype(np_type))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_slices_and_gaps(sdk, orc, dtype):
+    """An offset and row strides that are not whole vectors; a broadcast
+    (stride 0) batch dimension."""
+    x = orc.normal((90 * 131 + 7,), 92, 0, 0.0, 1.0, dtype)
+    tx = sdk.from_numpy(x)
+    for shape, strides, offset in [((77, 80), (1, 131), 7), ((66, 3, 88), (1, 5, 131), 3),
+                                   ((4, 70, 65), (0, 1, 100), 1), ((3, 66, 70), (1, 131, 17), 5)]:
+        idx = offset + sum(np.arange(n).reshape([-1 if i == d else 1 for i in range(len(shape))]) * s
+                           for d, (n, s) in enumerate(zip(shape, strides)))
+        ty = sdk.tensor(dtype, shape)
+        sdk.call(f"tensor_view_add_mul_{dtype}", tx, TensorView.make(shape, strides, offset), None, None, ty)
+        assert np.array_equal(ty.download(), x[idx])
