@@ -20,6 +20,7 @@
 // the end (acc / sum) rather than per weight, and the online rescaling
 // reorders the roundings of p; outputs therefore agree with the reference to
 // a few roundings of sum_j p_j |v_j|.
+#include "decode.hpp"
 #include "flash.hpp"
 #include "kern_common.hpp"
 #include "kernels.hpp"
@@ -372,6 +373,21 @@ SdpaArgs flash_args(const FlashPlan &p, const k::SdpaShape &sh, float scale, boo
     return a;
 }
 
+// The decode kernels' plan and arguments, or use == false. Without the
+// workspace for several parts the keys stay in one.
+DecodePlan decode_args(const k::SdpaShape &sh, bool aligned, bool f32, float scale, bool causal,
+                       void *workspace, size_t workspace_bytes, SdpaArgs *a) {
+    DecodePlan d = decode_plan(sh, aligned, f32, causal);
+    if (!d.use) return d;
+    if (d.parts > 1 && (workspace == nullptr || workspace_bytes < decode_workspace(d, sh))) d.parts = 1;
+    *a = flash_args(FlashPlan{}, sh, scale, causal, nullptr);
+    if (d.parts > 1) {
+        a->part_o = static_cast<float *>(workspace);
+        a->part_ml = reinterpret_cast<f32x4 *>(a->part_o + (size_t)d.parts * sh.batch * sh.q_heads * sh.q_len * sh.value_dim);
+    }
+    return d;
+}
+
 template <typename S, bool kAnyDim>
 hipError_t combine_splits(const SdpaArgs &a, const FlashPlan &p, const S *q, const S *k, const S *v,
                           const S *mask, S *out, hipStream_t s) {
@@ -461,6 +477,8 @@ hipError_t combine_splits(const SdpaArgs &a, const FlashPlan &p, const S *q, con
 namespace k {
 
 size_t sdpa_workspace_bytes(const SdpaShape &shape, bool f32, bool causal) {
+    const DecodePlan d = decode_plan(shape, true, f32, causal);
+    if (d.use) return decode_workspace(d, shape);
     const FlashPlan p = flash_plan(shape, true, f32, causal, true);
     return p.flash && p.max_parts > 1 ? partial_bytes(shape, p.max_parts) : 0;
 }
@@ -469,6 +487,9 @@ hipError_t sdpa_f32(const float *q, const float *k, const float *v, const float 
                     float *out, const SdpaShape &shape, float scale, bool causal,
                     void *workspace, size_t workspace_bytes, hipStream_t s) {
     const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15u) == 0;
+    SdpaArgs da;
+    const DecodePlan decode = decode_args(shape, aligned, true, scale, causal, workspace, workspace_bytes, &da);
+    if (decode.use) return launch_decode_f32(decode, q, k, v, mask, out, da, s);
     const FlashPlan plan = launch_plan(shape, aligned, true, causal, workspace_bytes, workspace);
     if (!plan.flash) return launch_sdpa<float>(q, k, v, mask, out, shape, scale, causal, s);
     const SdpaArgs a = flash_args(plan, shape, scale, causal, workspace);
@@ -492,6 +513,9 @@ hipError_t sdpa_f16(const uint16_t *q, const uint16_t *k, const uint16_t *v,
     auto h = [](const uint16_t *p) { return reinterpret_cast<const _Float16 *>(p); };
     _Float16 *o16 = reinterpret_cast<_Float16 *>(out);
     const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15u) == 0;
+    SdpaArgs da;
+    const DecodePlan decode = decode_args(shape, aligned, false, scale, causal, workspace, workspace_bytes, &da);
+    if (decode.use) return launch_decode_f16(decode, h(q), h(k), h(v), h(mask), o16, da, s);
     const FlashPlan plan = launch_plan(shape, aligned, false, causal, workspace_bytes, workspace);
     if (!plan.flash)
         return launch_sdpa<_Float16>(h(q), h(k), h(v), h(mask), o16, shape, scale, causal, s);
