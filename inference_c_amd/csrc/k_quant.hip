@@ -29,19 +29,13 @@
 // Bound: HBM bytes of the packed weights (1.0625 or 0.5625 bytes per weight).
 #include "kern_common.hpp"
 #include "kernels.hpp"
+#include "quant_common.hpp"
 
 #include <type_traits>
 
 namespace icsdk {
 namespace k {
 namespace {
-
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-
-template <bool kQ8> struct Fmt {
-    static constexpr uint32_t kBytes = kQ8 ? 34 : 18;
-};
 
 // Calls f(std::integral_constant<int, i>) for i = 0 .. N-1, unrolled.
 template <int N, int I = 0, typename F> __device__ inline void static_for(F &&f) {
@@ -50,8 +44,6 @@ template <int N, int I = 0, typename F> __device__ inline void static_for(F &&f)
         static_for<N, I + 1>(f);
     }
 }
-
-__device__ inline half2_t as_half2(uint32_t bits) { return __builtin_bit_cast(half2_t, bits); }
 
 // GEMV block arithmetic. Lane l of a chunk owns block l; the block starts at
 // an even byte offset `off` of the staged row, so the kWin 4-byte words read
@@ -147,58 +139,6 @@ __device__ inline void gemv_block(const uint8_t *chunk, uint32_t off, const Gemv
 #pragma unroll
         for (int r = 0; r < R; ++r) dot[r] = __builtin_fmaf(s1[r], 0.0625f, s0[r]);
     }
-}
-
-// One output by the reference's own chain (tensor_compute_cuda.cu:216-238):
-// sum = fmaf(x_k, scale_b * q_k, sum) over the blocks b of the row, then the
-// 32 values k of each, from 0. The fix-up for an output whose fast sum is
-// not finite. Finite x and finite scales keep every partial sum of the fast
-// kernels finite (at most ~2^30 for f16 operands), and a non-finite x makes
-// the reference's sum non-finite too, but the offset decode forms
-// x (q + offset) - offset x, so x = +-Inf gives Inf - Inf = NaN where the
-// reference's x * (scale q) gives +-Inf (NaN only for q = 0, a zero scale
-// or infinities of both signs). Running the reference's chain for those
-// outputs makes them equal to the reference's bit for bit. `xrow` is the
-// input row (16-byte aligned), `wrow` the packed weight row (2-byte
-// aligned). Rare: only rows with an infinity or NaN take it.
-template <bool kQ8>
-__device__ inline float reference_chain(const uint16_t *xrow, const uint8_t *wrow,
-                                        uint32_t blocks) {
-    constexpr uint32_t kBytes = Fmt<kQ8>::kBytes;
-    float sum = 0.0f;
-#pragma unroll 1
-    for (uint32_t b = 0; b < blocks; ++b) {
-        const uint16_t *blk = reinterpret_cast<const uint16_t *>(wrow + (uint64_t)b * kBytes);
-        uint16_t half_words[kBytes / 2];
-#pragma unroll
-        for (uint32_t i = 0; i < kBytes / 2; ++i) half_words[i] = blk[i];
-        const u32x4 *xp = reinterpret_cast<const u32x4 *>(xrow + (uint64_t)b * 32);
-        uint32_t xw[16];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const u32x4 t = xp[v];
-            xw[4 * v] = t.x;
-            xw[4 * v + 1] = t.y;
-            xw[4 * v + 2] = t.z;
-            xw[4 * v + 3] = t.w;
-        }
-        const float scale = (float)__builtin_bit_cast(_Float16, half_words[0]);
-#pragma unroll
-        for (uint32_t k = 0; k < 32; ++k) {
-            int q;
-            if constexpr (kQ8) {
-                const uint32_t byte = k;   // value byte k sits at block byte 2 + k
-                q = (int)(int8_t)(uint8_t)(half_words[1 + byte / 2] >> (8 * (byte & 1)));
-            } else {
-                const uint32_t byte = k & 15;
-                const uint8_t packed = (uint8_t)(half_words[1 + byte / 2] >> (8 * (byte & 1)));
-                q = (int)(k < 16 ? packed & 15 : packed >> 4) - 8;
-            }
-            const uint16_t xb = (uint16_t)(xw[k / 2] >> (16 * (k & 1)));
-            sum = __builtin_fmaf((float)__builtin_bit_cast(_Float16, xb), scale * (float)q, sum);
-        }
-    }
-    return sum;
 }
 
 // Grid: x = waves of O output rows (4 waves per block), y = groups of R
@@ -970,6 +910,10 @@ hipError_t linear_quant(const uint16_t *x, const uint8_t *w, uint16_t *y, size_t
     // 64 vs 52; Q4_0 2 rows 39 vs 44, 4 rows 52 vs 40). Its 32-bit offsets
     // bound `in`; past that every row takes the 1-row GEMV. Row groups per
     // launch stay within the grid's y limit.
+    if (rows > 16) {
+        const hipError_t e = quant_gemm(kQ8, x, w, y, rows, in, out, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     constexpr size_t kMaxGroups = 65535;
     const bool mma = rows > 2 && in <= (size_t{1} << 25);
     for (size_t r0 = 0; r0 < rows;) {
