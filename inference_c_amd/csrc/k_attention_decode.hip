@@ -48,8 +48,6 @@ namespace flash {
 namespace {
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4_2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef float f32x4_4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kDecodeWaves = 4;
 constexpr float kLog2e = 1.4426950408889634f;
