@@ -141,13 +141,13 @@ bool make_plan(hipblasLtHandle_t handle, GemmKind kind, hipDataType type, uint64
 bool gemm(GemmKind kind, TensorDType dtype, const void *x, const void *w, const void *bias,
           void *y, size_t rows, size_t inner, size_t cols, hipStream_t stream, char *error,
           size_t capacity) {
-    if (ICSDK_GEMV_LINEAR && kind == GemmKind::kLinear && rows <= k::kGemvMaxRows) {
-        // decode-sized linears stream the weights through a GEMV kernel
-        const hipError_t e = k::linear_gemv(dtype == TENSOR_DTYPE_F32, x, w, bias, y, rows, inner,
-                                            cols, stream);
+    if (ICSDK_GEMV_LINEAR && kind == GemmKind::kLinear) {
+        // few input rows and small sizes run on kernels of our own
+        const hipError_t e = k::linear_small(dtype == TENSOR_DTYPE_F32, x, w, bias, y, rows, inner,
+                                             cols, stream);
         if (e == hipSuccess) return true;
         if (e != hipErrorNotSupported) {
-            set_error(error, capacity, "GEMV launch failed: %s", hipGetErrorString(e));
+            set_error(error, capacity, "linear launch failed: %s", hipGetErrorString(e));
             return false;
         }
     }
