@@ -587,7 +587,8 @@ __global__ __launch_bounds__(BM * 2 * KS) void sdpa_flash_kernel(const _Float16 
         // wait for them leaves those in flight (and no branch lies between).
         // A 2-byte load per score, each behind its own bounds test, bound the
         // masked kernels (us, before -> now: 32q/8kv 2048 x 2048 D 128 308 -> 101,
-        // D 64 284 -> 77, 12 heads 1024 x 1024 D 64 77 -> 23; unmasked 14).
+        // D 64 284 -> 77; with the second key part that the freed registers
+        // allow, 12 heads 1024 x 1024 D 64 77 -> 16, unmasked 14).
         u32x4 mvec[kMask ? 4 : 1];
         if constexpr (kMask) {
             const _Float16 *mrow = mask + (size_t)(q_live ? qi : 0) * a.kl;

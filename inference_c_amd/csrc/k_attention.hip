@@ -423,24 +423,11 @@ hipError_t combine_splits(const SdpaArgs &a, const FlashPlan &p, const S *q, con
         else                                                                                       \
             hipLaunchKernelGGL((KERNEL<D, BM, false, false, KS>), grid, block, 0, s, Q, K, V, M, O, a);\
     } while (0)
-// two key parts: the raw-product variants only (the general variant would
-// not fit two waves per SIMD at D 128 and runs with one key part)
-#define ICSDK_FLASH_VARIANTS_KS2(KERNEL, D, Q, K, V, M, O)                                         \
-    do {                                                                                           \
-        if (split)                                                                                 \
-            hipLaunchKernelGGL((KERNEL<D, 128, false, true, 2>), grid, block, 0, s, Q, K, V, M, O, a); \
-        else                                                                                       \
-            hipLaunchKernelGGL((KERNEL<D, 128, false, false, 2>), grid, block, 0, s, Q, K, V, M, O, a);\
-    } while (0)
 // two-part blocks of 64 or 128 queries
 #define ICSDK_FLASH_VARIANTS_KS2_BM(KERNEL, D, Q, K, V, M, O)                                     \
     do {                                                                                           \
-        if (plan.bm == 64 && split)                                                                \
-            hipLaunchKernelGGL((KERNEL<D, 64, false, true, 2>), grid, block, 0, s, Q, K, V, M, O, a); \
-        else if (plan.bm == 64)                                                                    \
-            hipLaunchKernelGGL((KERNEL<D, 64, false, false, 2>), grid, block, 0, s, Q, K, V, M, O, a); \
-        else                                                                                       \
-            ICSDK_FLASH_VARIANTS_KS2(KERNEL, D, Q, K, V, M, O);                                    \
+        if (plan.bm == 64) ICSDK_FLASH_VARIANTS_KS(KERNEL, D, 64, 2, Q, K, V, M, O);               \
+        else ICSDK_FLASH_VARIANTS_KS(KERNEL, D, 128, 2, Q, K, V, M, O);                            \
     } while (0)
 // the f32 kernel: 64- or 128-query blocks, 64- or 128-query blocks with two
 // key parts per query group
@@ -495,7 +482,10 @@ hipError_t sdpa_f32(const float *q, const float *k, const float *v, const float 
     const SdpaArgs a = flash_args(plan, shape, scale, causal, workspace);
     const bool split = plan.max_parts > 1;
     const bool general = mask != nullptr;
-    const uint32_t ks = general ? 1 : plan.key_parts;
+    // with a mask a second key part pays from the second key tile on (its
+    // clamped mask loads cost more than a plain tile's: 16 x 8 heads 50 x 50
+    // D 64 f16 6.5 us, two parts 8.2)
+    const uint32_t ks = general && shape.kv_len <= plan.tk ? 1 : plan.key_parts;
     const dim3 grid((unsigned)(shape.batch * shape.q_heads * plan.items)), block(2 * plan.bm * ks);
     if (plan.any_dim) {
         const hipError_t status = launch_any_dim_f32({plan.dim, plan.bm, ks, general, split}, grid,
@@ -524,7 +514,7 @@ hipError_t sdpa_f16(const uint16_t *q, const uint16_t *k, const uint16_t *v,
     // the raw-product softmax needs scale > 0; other scales take the general
     // (mask) variant, whose mask may be null
     const bool general = mask != nullptr || !(scale > 0.0f);
-    const uint32_t ks = general ? 1 : plan.key_parts;
+    const uint32_t ks = general && shape.kv_len <= plan.tk ? 1 : plan.key_parts;
     const dim3 grid((unsigned)(shape.batch * shape.q_heads * plan.items)), block(2 * plan.bm * ks);
     if (plan.any_dim) {
         const hipError_t status = launch_any_dim_f16({plan.dim, plan.bm, ks, general, split}, grid,

@@ -32,26 +32,14 @@ namespace {
         return hipGetLastError();                                                              \
     } while (0)
 
-// without a mask only (two key parts)
-#define ICSDK_ANY_DIM_PLAIN(KERNEL, D, BM, KS)                                                 \
-    do {                                                                                       \
-        if (variant.split)                                                                     \
-            hipLaunchKernelGGL((KERNEL<D, BM, false, true, KS, true>), grid, block, 0, s, q,   \
-                               k, v, mask, out, a);                                            \
-        else                                                                                   \
-            hipLaunchKernelGGL((KERNEL<D, BM, false, false, KS, true>), grid, block, 0, s, q,  \
-                               k, v, mask, out, a);                                            \
-        return hipGetLastError();                                                              \
-    } while (0)
-
 template <int D>
 hipError_t launch_f16(const FlashVariant &variant, dim3 grid, dim3 block, hipStream_t s,
                       const _Float16 *q, const _Float16 *k, const _Float16 *v,
                       const _Float16 *mask, _Float16 *out, const SdpaArgs &a) {
     if constexpr (D <= 128) {
-        if (variant.key_parts == 2 && !variant.general) {
-            if (variant.bm == 64) ICSDK_ANY_DIM_PLAIN(sdpa_flash_kernel, D, 64, 2);
-            ICSDK_ANY_DIM_PLAIN(sdpa_flash_kernel, D, 128, 2);
+        if (variant.key_parts == 2) {
+            if (variant.bm == 64) ICSDK_ANY_DIM(sdpa_flash_kernel, D, 64, 2);
+            ICSDK_ANY_DIM(sdpa_flash_kernel, D, 128, 2);
         }
         if (variant.bm == 256) ICSDK_ANY_DIM(sdpa_flash_kernel, D, 256, 1);
     }
@@ -67,7 +55,6 @@ hipError_t launch_f32(const FlashVariant &variant, dim3 grid, dim3 block, hipStr
     ICSDK_ANY_DIM(sdpa_flash_f32_kernel, D, 64, 1);
 }
 
-#undef ICSDK_ANY_DIM_PLAIN
 #undef ICSDK_ANY_DIM
 
 }  // namespace
