@@ -131,6 +131,8 @@ def cpu_baseline(suite_results=None, step_kernels=None, reps=5):
     import numpy as np
     from oracle import Oracle, load_reference
     orc, ref = Oracle(), load_reference()
+    if ref is None:   # its sources are not on this machine
+        return {"value": None, "kind": "not measured: oracle/_ref/libref.so is not built"}
     err = ctypes.create_string_buffer(256)
     gpu = dict(suite_results or {})
     gpu.update(step_kernels or {})   # the step's own figures where it has them
