@@ -702,7 +702,12 @@ hipError_t launch_view(const S *x, const k::ViewArgs &v, const S *addend,
         // 64 x 64 tiles of vectors: both dims of at least 64 elements (the
         // scalar arguments hold dims, the x row stride, the offset and the
         // output row stride in 32 bits; the operands' rows run along last)
-        if (np >= kTile && nl >= kTile && np + kTile <= lim && nl + 4 * kTile <= lim &&
+        // An operand that is the output (y = view(x) + y) is read by the lane
+        // that writes its element; a tile that overlaps another one would
+        // read what that one has written.
+        const bool overlap = np % kTile != 0 || nl % kTile != 0;
+        const bool in_place = (addend && addend == y) || (mult && mult == y);
+        if (!(in_place && overlap) && np >= kTile && nl >= kTile && np + kTile <= lim && nl + 4 * kTile <= lim &&
             c.x_stride[last] > 0 && (uint64_t)c.x_stride[last] <= lim && v.offset <= lim &&
             plan.y_stride[p] <= lim && c.a_stride[last] <= 1 && c.m_stride[last] <= 1) {
             plan.tiles_p = (uint32_t)((np + kTile - 1) / kTile);

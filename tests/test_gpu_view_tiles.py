@@ -64,3 +64,23 @@ def test_slices_and_gaps(sdk, orc, dtype):
         ty = sdk.tensor(dtype, shape)
         sdk.call(f"tensor_view_add_mul_{dtype}", tx, TensorView.make(shape, strides, offset), None, None, ty)
         assert np.array_equal(ty.download(), x[idx])
+
+
+@pytest.mark.parametrize("shape", [(128, 192), (65, 64), (67, 129), (130, 4099), (3000, 1000)])
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("add,mul", [(True, False), (False, True), (True, True)])
+def test_output_is_an_operand(sdk, orc, shape, dtype, add, mul):
+    """y = view(x) + y, view(x) * y, (view(x) + y) * y: each element of y
+    enters once, as it was before the call."""
+    np_type = np.float16 if dtype == "f16" else np.float32
+    x = orc.normal(shape, 93, 0, 0.0, 1.0, dtype)
+    y = orc.normal(shape[::-1], 93, 1, 0.0, 1.0, dtype)
+    ty = sdk.from_numpy(y)
+    sdk.call(f"tensor_view_add_mul_{dtype}", sdk.from_numpy(x), TensorView.make(shape[::-1], (1, shape[1])),
+             ty if add else None, ty if mul else None, ty)
+    want = x.T.astype(np.float32)
+    if add:
+        want = want + y.astype(np.float32)
+    if mul:
+        want = want * y.astype(np.float32)
+    assert np.array_equal(ty.download(), want.astype(np_type))
