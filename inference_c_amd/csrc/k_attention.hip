@@ -463,11 +463,27 @@ hipError_t combine_splits(const SdpaArgs &a, const FlashPlan &p, const S *q, con
 
 namespace k {
 
-size_t sdpa_workspace_bytes(const SdpaShape &shape, bool f32, bool causal) {
-    const DecodePlan d = decode_plan(shape, true, f32, causal);
+// Calls that keep off the kernels whose second pass over a row reads q again,
+// or whose parts need scratch memory where the flash kernels of D 64 and 128
+// and the row kernel need none: an output in place of q, and a launch that a
+// graph records (a replay would use the scratch after it went back).
+struct Route {
+    bool in_place, captured;
+    Route(const void *q, const void *out, hipStream_t s) : in_place(q == out) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        captured = hipStreamIsCapturing(s, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
+    }
+    bool decode() const { return !in_place && !captured; }
+};
+
+size_t sdpa_workspace_bytes(const SdpaShape &shape, bool f32, bool causal, const void *q,
+                            const void *out, hipStream_t s) {
+    const Route route(q, out, s);
+    const DecodePlan d = decode_plan(shape, route.decode(), f32, causal);
     if (d.use) return decode_workspace(d, shape);
     const FlashPlan p = flash_plan(shape, true, f32, causal, true);
-    return p.flash && p.max_parts > 1 ? partial_bytes(shape, p.max_parts) : 0;
+    const bool split = p.flash && p.max_parts > 1 && !(p.any_dim && route.captured);
+    return split ? partial_bytes(shape, p.max_parts) : 0;
 }
 
 hipError_t sdpa_f32(const float *q, const float *k, const float *v, const float *mask,
@@ -475,7 +491,9 @@ hipError_t sdpa_f32(const float *q, const float *k, const float *v, const float 
                     void *workspace, size_t workspace_bytes, hipStream_t s) {
     const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15u) == 0;
     SdpaArgs da;
-    const DecodePlan decode = decode_args(shape, aligned, true, scale, causal, workspace, workspace_bytes, &da);
+    const Route route(q, out, s);
+    const DecodePlan decode = decode_args(shape, aligned && route.decode(), true, scale, causal, workspace,
+                                          workspace_bytes, &da);
     if (decode.use) return launch_decode_f32(decode, q, k, v, mask, out, da, s);
     const FlashPlan plan = launch_plan(shape, aligned, true, causal, workspace_bytes, workspace);
     if (!plan.flash) return launch_sdpa<float>(q, k, v, mask, out, shape, scale, causal, s);
@@ -504,10 +522,12 @@ hipError_t sdpa_f16(const uint16_t *q, const uint16_t *k, const uint16_t *v,
     _Float16 *o16 = reinterpret_cast<_Float16 *>(out);
     const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15u) == 0;
     SdpaArgs da;
-    const DecodePlan decode = decode_args(shape, aligned, false, scale, causal, workspace, workspace_bytes, &da);
+    const Route route(q, out, s);
+    const DecodePlan decode = decode_args(shape, aligned && route.decode(), false, scale, causal, workspace,
+                                          workspace_bytes, &da);
     if (decode.use) return launch_decode_f16(decode, h(q), h(k), h(v), h(mask), o16, da, s);
     const FlashPlan plan = launch_plan(shape, aligned, false, causal, workspace_bytes, workspace);
-    if (!plan.flash)
+    if (!plan.flash || (plan.any_dim && route.in_place))
         return launch_sdpa<_Float16>(h(q), h(k), h(v), h(mask), o16, shape, scale, causal, s);
     const SdpaArgs a = flash_args(plan, shape, scale, causal, workspace);
     const bool split = plan.max_parts > 1;
