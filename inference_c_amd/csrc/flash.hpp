@@ -347,13 +347,24 @@ __device__ inline void write_partial(const SdpaArgs &a, uint32_t split, size_t r
 // otherwise out = (sum_s w_s o_s) * (1 / sum_s w_s l_s) with w_s =
 // exp(m_s - M) (exp2 when the maxima are in log2 units). One thread per 8
 // output elements; kAnyDim: the last group of a row may hold only 4 (an f32
-// value dim of 4 mod 8).
+// value dim of 4 mod 8), and an f16 row takes a power of two of lanes, so that
+// it lies in one wave: the wave that does a row again stores all of it, and
+// no other wave may have a part of the same row to store. (The spare lanes
+// of 72 .. 96 wide rows: 16 lanes for 9 .. 12 groups.)
 //
 // kParts >= the launch's largest part count: every part's (m, l) and output
 // vectors are requested up front, unconditionally (a part index past the
 // row's own count reads its last part again, which stays in bounds, and is
 // left out of the sums), so a row costs one memory round trip; walking the
 // parts in a run-time loop waited for each part's loads in turn.
+template <typename S, bool kAnyDim> __host__ __device__ inline uint32_t combine_lanes(uint32_t vdim) {
+    const uint32_t groups = (vdim + 7) / 8;
+    if (!(kAnyDim && sizeof(S) == 2)) return groups;
+    uint32_t lanes = 1;
+    while (lanes < groups) lanes *= 2;
+    return lanes;   // at most 32 (value dims up to 256)
+}
+
 template <typename S, bool kLog2, int kParts, bool kAnyDim>
 __global__ __launch_bounds__(kBlock) void sdpa_combine_kernel(SdpaArgs a, S *__restrict__ out,
                                                               uint32_t bm, uint32_t tk,
@@ -362,13 +373,14 @@ __global__ __launch_bounds__(kBlock) void sdpa_combine_kernel(SdpaArgs a, S *__r
                                                               const S *mask) {
     const size_t rows = (size_t)a.batch * a.qh * a.ql;
     const uint32_t suffix = a.ql - first_row;
-    const uint32_t groups = (a.vdim + 7) / 8;
+    const uint32_t groups = (a.vdim + 7) / 8, lanes = combine_lanes<S, kAnyDim>(a.vdim);
     const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    const size_t last = (size_t)a.batch * a.qh * suffix * groups - 1;
-    const bool live = i <= last;
+    const size_t last = (size_t)a.batch * a.qh * suffix * lanes - 1;
+    const uint32_t lane_g = (uint32_t)(min(i, last) % lanes);
+    const bool live = i <= last && lane_g < groups;
     if (!(kAnyDim && sizeof(S) == 2) && !live) return;   // (the redo below takes whole waves)
-    const size_t srow = min(i, last) / groups;
-    const uint32_t g = (uint32_t)(min(i, last) % groups);
+    const size_t srow = min(i, last) / lanes;
+    const uint32_t g = min(lane_g, groups - 1);
     const uint32_t qi = first_row + (uint32_t)(srow % suffix);
     const size_t row = srow / suffix * a.ql + qi;
     const uint32_t splits = split_parts(

@@ -392,7 +392,7 @@ template <typename S, bool kAnyDim>
 hipError_t combine_splits(const SdpaArgs &a, const FlashPlan &p, const S *q, const S *k, const S *v,
                           const S *mask, S *out, hipStream_t s) {
     const uint32_t first_row = p.first_split * p.bm;
-    const size_t n = (size_t)a.batch * a.qh * (a.ql - first_row) * ((a.vdim + 7) / 8);
+    const size_t n = (size_t)a.batch * a.qh * (a.ql - first_row) * combine_lanes<S, kAnyDim>(a.vdim);
     const dim3 grid((unsigned)((n + kBlock - 1) / kBlock)), block(kBlock);
     // the part-count bucket: no row of this launch has more parts
     static_assert(kMaxKeyParts <= 8, "combine buckets");

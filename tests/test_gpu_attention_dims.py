@@ -88,3 +88,21 @@ def test_f32_nan_before_the_visible_key(sdk, orc, dim):
     k[0, 0, 7, 0] = np.nan
     got = run_device(sdk, q, k, v, mask, 0.1, False, "f32")
     assert np.isnan(got[0, 0, 5]).all()
+
+
+@pytest.mark.parametrize("dim", [40, 72, 80, 88, 96, 136, 248])
+def test_merged_rows_are_done_again_whole(sdk, orc, dim):
+    """Keys cut into parts, an infinite value that every row sees: the merge
+    does those rows again, each as a whole (a row of 9 to 12 groups of 8 once
+    lay in two waves, and the one that had nothing to do again stored its own
+    columns at any time). An output in place of the queries takes the row
+    kernel, whose outputs every column must equal, each time."""
+    q, k, v, _ = inputs(orc, (1, 2, 2, 40, 2000, dim, dim), "f16", 75, False)
+    v[0, :, 1000, dim - 1] = np.inf
+    tq, tk, tv = sdk.from_numpy(q), sdk.from_numpy(k), sdk.from_numpy(v)
+    sdk.call("tensor_sdpa_device_f16", tq, tk, tv, None, 0.1, 0, tq)
+    rows = tq.download()
+    assert np.isposinf(rows[..., dim - 1]).all()
+    for _ in range(4):
+        got = run_device(sdk, q, k, v, None, 0.1, False, "f16")
+        assert np.array_equal(got.view(np.uint16), rows.view(np.uint16))
