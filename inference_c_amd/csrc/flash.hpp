@@ -652,8 +652,12 @@ __global__ __launch_bounds__(BM * 2 * KS) void sdpa_flash_kernel(const _Float16 
             // turns st into s and uses sc = 1 (fma(s, 1, -m) == s - m). The
             // interior test is taken once per tile (inside the unrolled loop
             // it became one branch per score).
+            // kAnyDim keeps s in natural units and takes log2 e into sc: a mask
+            // of the type's lowest value leaves scores near -65504 with steps of
+            // 2^-8, the same in log2 units (-94502) with steps of 2^-7 (rows of
+            // such scores alone: relative error 1.57e-3, in natural units 1.14e-3).
             auto score = [&](float raw, float add, uint32_t kk, bool edge) {
-                float s = __builtin_fmaf(add, kLog2e, raw * scale2);
+                float s = kAnyDim ? raw * a.scale + add : __builtin_fmaf(add, kLog2e, raw * scale2);
                 if (edge && (kk >= a.kl || (a.causal && (uint64_t)kk > lane_last_key)))
                     s = neg_inf;
                 return s;
@@ -748,7 +752,7 @@ __global__ __launch_bounds__(BM * 2 * KS) void sdpa_flash_kernel(const _Float16 
                             sv[hblk][r] = score(st[hblk][r], (float)mq[hblk][r / 4][r % 4],
                                                 k0 + 32 * hblk + 8 * (r / 4) + 4 * half + r % 4, true);
                 }
-                softmax(sv, 1.0f);
+                softmax(sv, kAnyDim ? kLog2e : 1.0f);
             } else {
                 // raw products, scale2 > 0: keys out of range or past the
                 // causal limit become -inf in place

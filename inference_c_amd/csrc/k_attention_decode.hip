@@ -26,7 +26,7 @@
 //   out^T row m of MFMA j is column VE m + j (f16: the 8 keys' elements j
 //   are gathered by v_perm, one per two; f32: each MFMA takes one key per
 //   group). Columns past the head dim load column 0 again and are not stored.
-// Softmax as in the flash kernel: log2 units (f32: natural), lazy rescale, NaN
+// Softmax as in the flash kernel: log2 units (f32, masked f16: natural), lazy rescale, NaN
 // flag for rows that have seen nothing yet; f16 P is the pair hi + lo. Each
 // lane sums its own keys; lane groups meet at the end. Waves merge through
 // LDS, parts through sdpa_fold_kernel. A row with a finite sum and an output
@@ -152,8 +152,12 @@ __global__ __launch_bounds__(kDecodeWaves *kWave) void sdpa_decode_kernel(
     for (int j = 0; j < NJ; ++j) o[j] = f32x4{0, 0, 0, 0};
     float mx = neg_inf, sum = 0.0f;
     bool nan_seen = false;
-    const float unit = kHalf ? kLog2e : 1.0f;   // scores in log2 units (f16) or natural
-    const float scale = a.scale * unit;
+    // f16 scores are in log2 units, f32 and masked f16 scores in natural ones:
+    // near a mask's -65504 those have the finer steps (2^-8; -94502 has 2^-7), and
+    // `unit` then enters with the maximum's subtraction, in one fma. The maximum
+    // is kept in the units of exp2 (f16) or expf (f32).
+    constexpr float unit = kHalf && kMask ? kLog2e : 1.0f;
+    const float scale = kHalf && !kMask ? a.scale * kLog2e : a.scale;
 
     auto power = [](float x) { return kHalf ? __builtin_amdgcn_exp2f(x) : expf(x); };
     // the last key the lane's row sees
@@ -188,7 +192,7 @@ __global__ __launch_bounds__(kDecodeWaves *kWave) void sdpa_decode_kernel(
                 if constexpr (kHalf) {
                     const half8 mv = __builtin_bit_cast(half8, (u32x4)*reinterpret_cast<const u32x4_2 *>(mrow + first));
 #pragma unroll
-                    for (int i = 0; i < KEYS; ++i) p[i] = __builtin_fmaf((float)mv[i], unit, p[i]);
+                    for (int i = 0; i < KEYS; ++i) p[i] = p[i] + (float)mv[i];
                 } else {
                     const f32x4 mv = *reinterpret_cast<const f32x4_4 *>(mrow + first);
 #pragma unroll
@@ -197,7 +201,7 @@ __global__ __launch_bounds__(kDecodeWaves *kWave) void sdpa_decode_kernel(
             } else {
 #pragma unroll
                 for (int i = 0; i < KEYS; ++i)
-                    if (first + i < a.kl) p[i] = __builtin_fmaf((float)mrow[first + i], unit, p[i]);
+                    if (first + i < a.kl) p[i] = p[i] + (float)mrow[first + i];
             }
         }
         if (key0 + kTileKeys > a.kl || a.causal) {
@@ -207,6 +211,7 @@ __global__ __launch_bounds__(kDecodeWaves *kWave) void sdpa_decode_kernel(
         float big = neg_inf;
 #pragma unroll
         for (int i = 0; i < KEYS; ++i) big = fmaxf(big, p[i]);
+        big *= unit;
         // f16: the running maximum moves only when a row's grows by more than
         // 2^kLazyLog2 (p stays within f16)
         if (__builtin_amdgcn_ballot_w64(big > mx + (kHalf ? kLazyLog2 : 0.0f)) != 0) {
@@ -227,7 +232,7 @@ __global__ __launch_bounds__(kDecodeWaves *kWave) void sdpa_decode_kernel(
         float add = 0.0f;
 #pragma unroll
         for (int i = 0; i < KEYS; ++i) {
-            p[i] = none ? 0.0f : power(p[i] - mx);
+            p[i] = none ? 0.0f : power(kHalf && kMask ? __builtin_fmaf(p[i], unit, -mx) : p[i] - mx);
             add += p[i];
         }
         sum += add;

@@ -32,3 +32,28 @@ def test_masks_of_any_row_length(sdk, orc, dtype, dim, lq, lk, causal):
     assert np.isfinite(got).all()
     rows = [i for i in range(lq) if i != 9]
     check(got[:, :, rows], want[:, :, rows], weight[:, :, rows], dtype, f"{dim} {lq} {lk} {causal}")
+
+
+# batch, q heads, kv heads, q len, kv len, head dim: few rows packed (whole and
+# in parts), key tiles whole and in parts
+@pytest.mark.parametrize("shape", [(8, 8, 2, 4, 300, 64), (4, 8, 2, 4, 2000, 128), (4, 8, 2, 4, 600, 72),
+                                   (4, 8, 2, 4, 2000, 200), (1, 4, 2, 130, 600, 72), (1, 4, 4, 70, 2000, 96),
+                                   (2, 4, 2, 150, 700, 200)])
+def test_rows_of_the_lowest_value(sdk, orc, shape):
+    """f16 rows whose keys all carry the type's lowest value. In f32 such a
+    score, about -65504, is rounded to steps of 2^-8: errors uniform within
+    2^-9, so the weights are 2^-9 / sqrt(3) off, and the outputs (sums of
+    values of mean zero) as much, beside their own rounding, at most
+    2^-11 / sqrt(3). A tenth over that; twice the step (scores times log2 e,
+    past 65536) gives 1.56e-3."""
+    b, h, kh, lq, lk, dim = shape
+    q, k, v, _ = inputs(orc, (b, h, kh, lq, lk, dim, dim), "f16", 92, False)
+    mask = np.full((lq, lk), np.finfo(np.float16).min, np.float16)
+    scale = 1.0 / np.sqrt(dim)
+    got = run_device(sdk, q, k, v, mask, scale, False, "f16").astype(np.float64)
+    k64, v64 = (np.repeat(a.astype(np.float64), h // kh, axis=1) for a in (k, v))
+    s = np.matmul(q.astype(np.float64), k64.transpose(0, 1, 3, 2)) * np.float64(np.float32(scale))
+    p = np.exp(s - s.max(-1, keepdims=True))     # (the same mask everywhere)
+    want = np.matmul(p / p.sum(-1, keepdims=True), v64)
+    error = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert error <= 1.1 * np.hypot(2.0 ** -9, 2.0 ** -11) / np.sqrt(3.0), error
