@@ -33,8 +33,14 @@ void set_error(char *error, size_t capacity, const char *format, ...) {
     va_end(args);
 }
 
+// A failed runtime call also leaves its error as the thread's last one, which
+// the check after the next kernel launch would report as that launch's. Every
+// failure that is answered here (by a message or by a fallback) takes it out.
+void forget_error() { (void)hipGetLastError(); }
+
 bool hip_ok(hipError_t status, const char *what, char *error, size_t capacity) {
     if (status == hipSuccess) return true;
+    forget_error();
     set_error(error, capacity, "%s: %s", what, hipGetErrorString(status));
     return false;
 }
@@ -117,7 +123,10 @@ void *scratch_acquire(size_t bytes) {
         }
     }
     void *p = nullptr;
-    if (hipMalloc(&p, c) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, c) != hipSuccess) {
+        forget_error();   // the caller runs without scratch memory
+        return nullptr;
+    }
     return p;
 }
 
@@ -153,7 +162,10 @@ void *weight_cache_get(const void *host, size_t bytes) {
         return found->second.second == bytes ? found->second.first : nullptr;
     bind_device();
     void *device = nullptr;
-    if (hipMalloc(&device, bytes) != hipSuccess) return nullptr;
+    if (hipMalloc(&device, bytes) != hipSuccess) {
+        forget_error();
+        return nullptr;
+    }
     if (!pinned_to_device(device, host, bytes, state().stream, nullptr, 0)) {
         (void)hipStreamSynchronize(state().stream);
         (void)hipFree(device);
@@ -191,8 +203,10 @@ uint32_t *host_word_acquire() {
         // coherent: a kernel's store is not held in a device cache; slabs stay
         // allocated for the life of the process
         if (hipHostMalloc(&slab, kWordsPerSlab * sizeof(uint32_t),
-                          hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+                          hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+            forget_error();
             return nullptr;
+        }
         for (size_t i = 0; i < kWordsPerSlab; ++i)
             free_words.push_back(static_cast<uint32_t *>(slab) + i);
     }

@@ -47,6 +47,7 @@ public:
                 hipEventCreateWithFlags(&c->done, hipEventDisableTiming) != hipSuccess) {
                 if (c->host) (void)hipHostFree(c->host);
                 delete c;
+                forget_error();
                 set_error(error, capacity, "pinned staging: cannot allocate page-locked memory");
                 return false;
             }

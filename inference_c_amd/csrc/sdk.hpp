@@ -24,6 +24,9 @@ int sdk_device();
 // than the initialising one may start on another device).
 void bind_device();
 
+// Clears the calling thread's last HIP error after a failure that was answered.
+void forget_error();
+
 // status == hipSuccess, or a message "<what>: <hip error text>".
 bool hip_ok(hipError_t status, const char *what, char *error, size_t capacity);
 

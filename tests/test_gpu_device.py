@@ -161,3 +161,16 @@ def test_host_slots_from_several_threads(sdk, orc):
     y = np.empty_like(inputs[0][0])
     assert fn(inputs[0][0].ctypes.data, inputs[0][1].ctypes.data, y.ctypes.data, sizes[0])
     assert np.array_equal(y.view(np.uint16), wants[0].view(np.uint16))
+
+
+def test_calls_after_a_failed_creation(sdk, orc):
+    """A tensor that device memory does not hold is refused with a message, and
+    the next call is not refused for it."""
+    from inference_c_amd.sdk import SdkError
+    x = orc.normal((3, 70001), 84, 0, 0.0, 1.0, "f32")
+    tx, ty = sdk.from_numpy(x), sdk.tensor("f32", x.shape)
+    for _ in range(2):
+        with pytest.raises(SdkError, match="out of memory"):
+            sdk.tensor("f32", (1 << 48,))
+        sdk.call("tensor_softmax_f32", tx, 0, ty)
+        assert np.allclose(ty.download().sum(-1), 1.0, atol=1e-4)
