@@ -73,7 +73,7 @@ int host_run(const T *q, const T *k, const T *v, const T *mask, T *out, size_t b
     const void *pm = mask ? st.in(mask, c.mask * sizeof(T)) : nullptr;
     void *po = st.out(out, c.out * sizeof(T));
     if (st.failed()) return 0;
-    const size_t ws_want = k::sdpa_workspace_bytes(shape, sizeof(T) == 4, causal != 0, pq, po, st.stream());
+    const size_t ws_want = k::sdpa_workspace_bytes(shape, sizeof(T) == 4, causal != 0, pq, po);
     ScratchBlock workspace(ws_want);
     const size_t ws_bytes = workspace.get() ? ws_want : 0;
     hipError_t status;
@@ -167,10 +167,8 @@ int sdpa_device(TensorDType dtype, const TensorBuffer *q, const TensorBuffer *k,
     auto dev = [](const TensorBuffer *t) -> void * {
         return t ? tensor_buffer_device_handle_internal(t) : nullptr;
     };
-    // split-key partials live in a pool block, returned right after the
-    // launches (later users of the block enqueue behind them on the stream)
-    const size_t ws_want = k::sdpa_workspace_bytes(shape, dtype == TENSOR_DTYPE_F32, causal != 0, dev(q), dev(out),
-                                                   sdk_stream());
+    // split-key partials
+    const size_t ws_want = k::sdpa_workspace_bytes(shape, dtype == TENSOR_DTYPE_F32, causal != 0, dev(q), dev(out));
     ScratchBlock workspace(ws_want);
     const size_t ws_bytes = workspace.get() ? ws_want : 0;
     const hipError_t status =

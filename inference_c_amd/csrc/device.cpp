@@ -16,6 +16,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <map>
+#include <new>
 #include <vector>
 
 struct TensorDeviceBuffer {
@@ -136,12 +137,103 @@ void scratch_release(void *ptr, size_t bytes) {
     pool.emplace(size_class(bytes), ptr);
 }
 
+namespace {
+
+// Blocks of graphs. Those that have come back serve later captures. Never
+// destroyed: a graph may outlive this file's static objects.
+struct GraphBlocks {
+    std::mutex mutex;
+    std::multimap<size_t, void *> free;
+};
+GraphBlocks &graph_blocks() {
+    static GraphBlocks *g = new GraphBlocks;
+    return *g;
+}
+struct GraphBlock {
+    void *ptr;
+    size_t size;
+};
+// A graph's last owner is gone (no HIP calls here: the runtime forbids them).
+void give_back(void *p) {
+    GraphBlock *b = static_cast<GraphBlock *>(p);
+    {
+        std::lock_guard<std::mutex> lock(graph_blocks().mutex);
+        graph_blocks().free.emplace(b->size, b->ptr);
+    }
+    delete b;
+}
+
+}  // namespace
+
+Recording sdk_recording() {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(state().stream, &status) != hipSuccess) {
+        forget_error();
+        return Recording::kBroken;
+    }
+    return status == hipStreamCaptureStatusNone     ? Recording::kNo
+           : status == hipStreamCaptureStatusActive ? Recording::kYes
+                                                    : Recording::kBroken;
+}
+
+void *graph_scratch_acquire(size_t bytes) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    hipGraph_t graph = nullptr;
+    if (hipStreamGetCaptureInfo_v2(state().stream, &status, &id, &graph, nullptr, nullptr) != hipSuccess ||
+        status != hipStreamCaptureStatusActive || graph == nullptr) {
+        forget_error();
+        return nullptr;
+    }
+    const size_t c = size_class(bytes);
+    auto *block = new (std::nothrow) GraphBlock{nullptr, c};
+    if (block == nullptr) return nullptr;
+    {
+        std::lock_guard<std::mutex> lock(graph_blocks().mutex);
+        auto found = graph_blocks().free.find(c);
+        if (found != graph_blocks().free.end()) {
+            block->ptr = found->second;
+            graph_blocks().free.erase(found);
+        }
+    }
+    if (block->ptr == nullptr) {
+        // an allocation is no part of the graph; modes other than relaxed refuse it
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool switched = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        const bool failed = hipMalloc(&block->ptr, c) != hipSuccess;
+        if (switched) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (failed) {
+            forget_error();
+            delete block;
+            return nullptr;
+        }
+    }
+    void *const ptr = block->ptr;   // (the block may be gone once the graph owns it)
+    hipUserObject_t owner = nullptr;
+    if (hipUserObjectCreate(&owner, block, give_back, 1, hipUserObjectNoDestructorSync) != hipSuccess) {
+        forget_error();
+        give_back(block);
+        return nullptr;
+    }
+    if (hipGraphRetainUserObject(graph, owner, 1, hipGraphUserObjectMove) != hipSuccess) {
+        forget_error();
+        (void)hipUserObjectRelease(owner, 1);   // gives the block back
+        return nullptr;
+    }
+    return ptr;
+}
+
 void scratch_clear() {
     std::vector<void *> blocks;
     {
         std::lock_guard<std::mutex> lock(pool_mutex);
         for (auto &entry : pool) blocks.push_back(entry.second);
         pool.clear();
+    }
+    {
+        std::lock_guard<std::mutex> lock(graph_blocks().mutex);
+        for (auto &entry : graph_blocks().free) blocks.push_back(entry.second);
+        graph_blocks().free.clear();
     }
     if (blocks.empty() || !state().ready) return;
     bind_device();

@@ -182,8 +182,6 @@ bool gemm(GemmKind kind, TensorDType dtype, const void *x, const void *w, const 
             return false;
         }
     }
-    // the workspace comes from the staging pool; later users of the block
-    // enqueue on the same stream, after this GEMM
     ScratchBlock workspace(plan.workspace);
     if (plan.workspace != 0 && workspace.get() == nullptr) {
         set_error(error, capacity, "out of device memory for the GEMM workspace");

@@ -24,6 +24,7 @@
 #include "flash.hpp"
 #include "kern_common.hpp"
 #include "kernels.hpp"
+#include "sdk.hpp"
 
 #include <algorithm>
 
@@ -463,27 +464,26 @@ hipError_t combine_splits(const SdpaArgs &a, const FlashPlan &p, const S *q, con
 
 namespace k {
 
-// Calls that keep off the kernels whose second pass over a row reads q again,
-// or whose parts need scratch memory where the flash kernels of D 64 and 128
-// and the row kernel need none: an output in place of q, and a launch that a
-// graph records (a replay would use the scratch after it went back).
-struct Route {
-    bool in_place, captured;
-    Route(const void *q, const void *out, hipStream_t s) : in_place(q == out) {
-        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        captured = hipStreamIsCapturing(s, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
-    }
-    bool decode() const { return !in_place && !captured; }
-};
-
+// An output in place of q keeps off the kernels that may do a row again, which
+// reads its q a second time: the decode kernels, and the f16 flash kernels of
+// other head dims than 64 and 128.
+//
+// A call that a graph records takes the same kernels as one that runs. At D 64
+// and 128 its key parts hold memory of the graph's own; at other head dims the
+// keys stay in one part, so such a graph holds one kernel and no memory
+// (decode kernels with one part against flash kernels with one, us: f16 32q/8kv
+// over 2048 keys D 128 22 against 33, 16q/4kv D 80 26 against 32, f32 59
+// against 238; never slower at 16 shapes of either type).
 size_t sdpa_workspace_bytes(const SdpaShape &shape, bool f32, bool causal, const void *q,
-                            const void *out, hipStream_t s) {
-    const Route route(q, out, s);
-    const DecodePlan d = decode_plan(shape, route.decode(), f32, causal);
+                            const void *out) {
+    const bool in_place = q == out;
+    const bool whole_dims = shape.head_dim == shape.value_dim && (shape.head_dim == 64 || shape.head_dim == 128);
+    if (!whole_dims && sdk_recording() != Recording::kNo) return 0;
+    const DecodePlan d = decode_plan(shape, !in_place, f32, causal);
     if (d.use) return decode_workspace(d, shape);
     const FlashPlan p = flash_plan(shape, true, f32, causal, true);
-    const bool split = p.flash && p.max_parts > 1 && !(p.any_dim && route.captured);
-    return split ? partial_bytes(shape, p.max_parts) : 0;
+    if (!p.flash || p.max_parts == 1 || (in_place && p.any_dim && !f32)) return 0;
+    return partial_bytes(shape, p.max_parts);
 }
 
 hipError_t sdpa_f32(const float *q, const float *k, const float *v, const float *mask,
@@ -491,8 +491,7 @@ hipError_t sdpa_f32(const float *q, const float *k, const float *v, const float 
                     void *workspace, size_t workspace_bytes, hipStream_t s) {
     const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15u) == 0;
     SdpaArgs da;
-    const Route route(q, out, s);
-    const DecodePlan decode = decode_args(shape, aligned && route.decode(), true, scale, causal, workspace,
+    const DecodePlan decode = decode_args(shape, aligned && q != out, true, scale, causal, workspace,
                                           workspace_bytes, &da);
     if (decode.use) return launch_decode_f32(decode, q, k, v, mask, out, da, s);
     const FlashPlan plan = launch_plan(shape, aligned, true, causal, workspace_bytes, workspace);
@@ -522,12 +521,11 @@ hipError_t sdpa_f16(const uint16_t *q, const uint16_t *k, const uint16_t *v,
     _Float16 *o16 = reinterpret_cast<_Float16 *>(out);
     const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15u) == 0;
     SdpaArgs da;
-    const Route route(q, out, s);
-    const DecodePlan decode = decode_args(shape, aligned && route.decode(), false, scale, causal, workspace,
+    const DecodePlan decode = decode_args(shape, aligned && q != out, false, scale, causal, workspace,
                                           workspace_bytes, &da);
     if (decode.use) return launch_decode_f16(decode, h(q), h(k), h(v), h(mask), o16, da, s);
     const FlashPlan plan = launch_plan(shape, aligned, false, causal, workspace_bytes, workspace);
-    if (!plan.flash || (plan.any_dim && route.in_place))
+    if (!plan.flash || (plan.any_dim && q == out))
         return launch_sdpa<_Float16>(h(q), h(k), h(v), h(mask), o16, shape, scale, causal, s);
     const SdpaArgs a = flash_args(plan, shape, scale, causal, workspace);
     const bool split = plan.max_parts > 1;

@@ -583,13 +583,6 @@ inline Cut cut_row(size_t vectors) {
     return c;
 }
 
-// Scratch memory cannot be taken from the pool for a launch that a graph
-// records: a replay would use it after it went back.
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
-}
-
 struct Plan {
     Shape shape;
     Cut cut;
@@ -597,7 +590,7 @@ struct Plan {
     bool ok;
 };
 
-template <typename S> Plan plan_row(size_t rows, size_t width, hipStream_t s) {
+template <typename S> Plan plan_row(size_t rows, size_t width) {
     constexpr size_t E = Vec16<S>::N;
     Plan p{{0, 0}, {0, 0}, 0, false};
     if (width < E || width > 0xfffffff0u) return p;
@@ -606,7 +599,7 @@ template <typename S> Plan plan_row(size_t rows, size_t width, hipStream_t s) {
     if (p.shape.t != 0) {
         p.blocks = blocks_for(p.shape, rows);
     } else {
-        if (capturing(s)) return p;
+        if (sdk_recording() != Recording::kNo) return p;   // one kernel and no memory in a graph
         p.cut = cut_row(vectors);
         p.blocks = rows * p.cut.parts;
     }
@@ -644,7 +637,7 @@ template <typename S> Plan plan_row(size_t rows, size_t width, hipStream_t s) {
 template <typename S>
 hipError_t rms_norm(const S *x, const S *residual, S *sum_out, const S *w, S *y, size_t rows,
                     size_t width, float eps, hipStream_t s) {
-    const Plan p = plan_row<S>(rows, width, s);
+    const Plan p = plan_row<S>(rows, width);
     if (!p.ok) return hipErrorNotSupported;
     const dim3 grid((unsigned)p.blocks);
 #define ICSDK_CASE(T, NV)                                                                        \
@@ -676,7 +669,7 @@ hipError_t rms_norm(const S *x, const S *residual, S *sum_out, const S *w, S *y,
 template <typename S>
 hipError_t layer_norm(const S *x, const S *scale, const S *bias, S *y, size_t rows, size_t width,
                       float eps, hipStream_t s) {
-    const Plan p = plan_row<S>(rows, width, s);
+    const Plan p = plan_row<S>(rows, width);
     if (!p.ok) return hipErrorNotSupported;
     const dim3 grid((unsigned)p.blocks);
 #define ICSDK_CASE(T, NV)                                                                          \
@@ -704,7 +697,7 @@ hipError_t layer_norm(const S *x, const S *scale, const S *bias, S *y, size_t ro
 template <typename S>
 hipError_t softmax(const S *x, S *y, size_t rows, size_t width, size_t q_len,
                    size_t causal_offset, hipStream_t s) {
-    const Plan p = plan_row<S>(rows, width, s);
+    const Plan p = plan_row<S>(rows, width);
     if (!p.ok) return hipErrorNotSupported;
     const dim3 grid((unsigned)p.blocks);
 #define ICSDK_CASE(T, NV)                                                                       \
@@ -726,7 +719,7 @@ hipError_t softmax(const S *x, S *y, size_t rows, size_t width, size_t q_len,
 
 template <typename S, bool kMax>
 hipError_t reduce(const S *x, float *y, size_t rows, size_t width, hipStream_t s) {
-    const Plan p = plan_row<S>(rows, width, s);
+    const Plan p = plan_row<S>(rows, width);
     if (!p.ok) return hipErrorNotSupported;
     const dim3 grid((unsigned)p.blocks);
 #define ICSDK_CASE(T, NV)                                                                       \

@@ -135,9 +135,9 @@ struct SdpaShape {
 };
 // `workspace` (may be null) lets the flash path split the key range of long
 // query blocks over several blocks: sdpa_workspace_bytes bytes (of the same
-// shape, q, out and stream), 0 when the call would not split.
+// shape, q and out), 0 when the call would not split.
 size_t sdpa_workspace_bytes(const SdpaShape &shape, bool f32, bool causal, const void *q,
-                            const void *out, hipStream_t s);
+                            const void *out);
 hipError_t sdpa_f32(const float *q, const float *k, const float *v, const float *mask,
                     float *out, const SdpaShape &shape, float scale, bool causal,
                     void *workspace, size_t workspace_bytes, hipStream_t s);

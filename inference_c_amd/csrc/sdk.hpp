@@ -31,7 +31,8 @@ void forget_error();
 bool hip_ok(hipError_t status, const char *what, char *error, size_t capacity);
 
 // Device staging memory for host-storage operands, reused across calls.
-// Blocks are cached by size class until scratch_clear().
+// Blocks are cached by size class until scratch_clear(), which also frees
+// the graph blocks that have come back.
 void *scratch_acquire(size_t bytes);
 void scratch_release(void *ptr, size_t bytes);
 void scratch_clear();
@@ -64,24 +65,42 @@ private:
     uint32_t *word_;
 };
 
-// A pool block held for the duration of one call (none for zero bytes).
-// Returning it to the pool right after the launches is safe: every later
-// user of the block enqueues on the same SDK stream, after this call's
-// kernels.
+// Whether launches on the SDK stream run now, are recorded into a graph, or
+// neither (a capture that has failed).
+enum class Recording { kNo, kYes, kBroken };
+Recording sdk_recording();
+
+// Device memory for launches that the graph being captured on the SDK stream
+// records: it belongs to that graph and goes back when the graph and every
+// executable made of it are destroyed, which the program does when no replay
+// is running. Never shared with calls outside the graph. nullptr when there
+// is none.
+void *graph_scratch_acquire(size_t bytes);
+
+// Scratch memory for one call (none for zero bytes). Outside a capture a pool
+// block, returned right after the launches: every later user of the block
+// enqueues on the same SDK stream, after this call's kernels. In a capture a
+// block of the graph's own: a replay runs long after the call, when a pool
+// block would be another call's, or freed.
 class ScratchBlock {
 public:
-    explicit ScratchBlock(size_t bytes)
-        : bytes_(bytes), ptr_(bytes == 0 ? nullptr : scratch_acquire(bytes)) {}
+    explicit ScratchBlock(size_t bytes) : bytes_(bytes) {
+        if (bytes == 0) return;
+        const Recording r = sdk_recording();
+        pooled_ = r == Recording::kNo;
+        ptr_ = pooled_ ? scratch_acquire(bytes) : r == Recording::kYes ? graph_scratch_acquire(bytes) : nullptr;
+    }
     ScratchBlock(const ScratchBlock &) = delete;
     ScratchBlock &operator=(const ScratchBlock &) = delete;
     ~ScratchBlock() {
-        if (ptr_ != nullptr) scratch_release(ptr_, bytes_);
+        if (ptr_ != nullptr && pooled_) scratch_release(ptr_, bytes_);
     }
     void *get() const { return ptr_; }
 
 private:
     size_t bytes_;
-    void *ptr_;
+    bool pooled_ = true;
+    void *ptr_ = nullptr;
 };
 
 // Partial-result buffer of the two-pass grid reductions. The launches of one
