@@ -249,6 +249,9 @@ FlashPlan flash_plan(const k::SdpaShape &sh, bool aligned, bool f32, bool causal
     else p.bm = 64;
     p.tk = f32 ? 32 : 64;
     p.qblocks = (uint32_t)((sh.q_len + p.bm - 1) / p.bm);
+    // more work-items than a launch holds (2^23 heads of a few queries with 512
+    // threads each): the row kernel
+    if (bhs * p.qblocks * 2 * p.bm * p.key_parts > 0xffffffffull) return FlashPlan{};
     p.items = p.qblocks;
     p.first_split = p.qblocks;
     p.xcd_heads = (sh.batch * sh.kv_heads) % 8 == 0;

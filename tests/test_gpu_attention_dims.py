@@ -106,3 +106,13 @@ def test_merged_rows_are_done_again_whole(sdk, orc, dim):
     for _ in range(4):
         got = run_device(sdk, q, k, v, None, 0.1, False, "f16")
         assert np.array_equal(got.view(np.uint16), rows.view(np.uint16))
+
+
+def test_more_heads_than_a_flash_launch_holds(sdk):
+    """2^23 heads of one query and one key: the output is the value row."""
+    shape = (1 << 20, 8, 1, 8)
+    v = (np.arange(1 << 26, dtype=np.uint32) % 2039).astype(np.float16).reshape(shape)
+    tq = tk = sdk.from_numpy(np.ones(shape, np.float16))
+    out = sdk.tensor("f16", shape)
+    sdk.call("tensor_sdpa_device_f16", tq, tk, sdk.from_numpy(v), None, 0.1, 0, out)
+    assert np.array_equal(out.download(), v)
