@@ -23,9 +23,11 @@
 //             along p, staged through LDS (swizzled or padded against bank
 //             conflicts) and written along the innermost dimension, so both
 //             HBM streams stay coalesced: 64x64 tiles in 16-byte vectors of
-//             any alignment where both dimensions have 64 elements, else
-//             tiles of about 4096 elements shaped to the smaller one;
-//   scalar  - anything else: one element per lane.
+//             any alignment where both dimensions have 64 elements (whole
+//             aligned vectors also with fewer), else tiles of about 4096 or
+//             1024 elements shaped to the smaller one;
+//   scalar  - anything else, and transposes that would leave a tile mostly
+//             empty: one element per lane.
 #include "kern_common.hpp"
 #include "kernels.hpp"
 
@@ -268,6 +270,14 @@ bool short_plan(const Coalesced &c, uint64_t x_offset, uint64_t n, ShortPlan *pl
 
 // ---- scalar path -------------------------------------------------------------
 
+// The product as the f32 value it is. (The compiler otherwise folds a f32
+// multiply and its conversion to f16 into v_fma_mixlo_f16, which rounds once:
+// another result at ties.)
+template <typename S> __device__ inline float rounded_f32(float v) {
+    if constexpr (sizeof(S) == 2) asm("" : "+v"(v));
+    return v;
+}
+
 struct ScalarPlan {
     int rank;
     uint64_t shape[kMaxRank];
@@ -297,7 +307,7 @@ __global__ __launch_bounds__(kBlock) void view_scalar_kernel(const S *__restrict
         }
         float r = Elem<S>::load(x[xo]);
         if (addend) r = r + Elem<S>::load(addend[ao]);
-        if (mult) r = r * Elem<S>::load(mult[mo]);
+        if (mult) r = rounded_f32<S>(r * Elem<S>::load(mult[mo]));
         y[i] = Elem<S>::store(r);
     }
 }
@@ -324,14 +334,6 @@ struct TilePlan {
     uint32_t tiles_p, tiles_l;
     FastDiv tile_p, tile_l;         // the adaptive tile's extents
 };
-
-// The product as the f32 value it is. (The compiler otherwise folds a f32
-// multiply and its conversion to f16 into v_fma_mixlo_f16, which rounds once:
-// another result at ties.)
-template <typename S> __device__ inline float rounded_f32(float v) {
-    if constexpr (sizeof(S) == 2) asm("" : "+v"(v));
-    return v;
-}
 
 // Where a batch starts in each operand.
 struct BatchBase {
@@ -421,10 +423,10 @@ __global__ __launch_bounds__(kBlock) void view_tile_kernel(const S *__restrict__
 // stored at any element alignment. A block takes kTiles tiles along the last dim: two for f16 where
 // that still leaves 1024 blocks, else one (f16 with an addend, one / two /
 // four tiles: [3000, 3000] 13.7 / 10.0 / 11.3 us, [8192, 8192] 48.9 / 47.0 /
-// 47.9, [4096, 4096] 13.4 / 15.0 / 16.4). kGuarded: the form for f16 whole
-// aligned vectors without operands: bounds tests instead of the overlap,
-// four tiles, each load waited for before the next, which is the faster one
-// there ([4096, 4000] 11.6 us against 12.7-12.8, [64, 512, 512] 12.4 against
+// 47.9, [4096, 4096] 13.4 / 15.0 / 16.4). kGuarded: the form for whole
+// aligned vectors without operands: bounds tests instead of the overlap (the
+// launcher says where), f16 with four tiles, each load waited for before the
+// next, which is the faster one there ([4096, 4000] 11.6 us against 12.7-12.8, [64, 512, 512] 12.4 against
 // 13.2-15.6). Operands enter as a vector along the last dim or as one element per
 // output row (OperandKind), loaded before the barrier. Against the
 // one-element-per-lane tiles: f16 [4097, 4095] 30.0 -> 21.4 us, [4096,
@@ -699,26 +701,51 @@ hipError_t launch_view(const S *x, const k::ViewArgs &v, const S *addend,
         const uint64_t np = c.shape[p], nl = c.shape[last], lim = 0xffffffffull;
         const int ka = !addend ? kNone : c.a_stride[last] != 0 ? kVector : kScalar;
         const int km = !mult ? kNone : c.m_stride[last] != 0 ? kVector : kScalar;
-        // 64 x 64 tiles of vectors: both dims of at least 64 elements (the
-        // scalar arguments hold dims, the x row stride, the offset and the
-        // output row stride in 32 bits; the operands' rows run along last)
+        // 64 x 64 tiles of vectors (the scalar arguments hold dims, the x row
+        // stride, the offset and the output row stride in 32 bits; the
+        // operands' rows run along last)
+        const bool fits32 = np + kTile <= lim && nl + 4 * kTile <= lim && c.x_stride[last] > 0 &&
+                            (uint64_t)c.x_stride[last] <= lim && v.offset <= lim && plan.y_stride[p] <= lim;
         // An operand that is the output (y = view(x) + y) is read by the lane
         // that writes its element; a tile that overlaps another one would
         // read what that one has written.
+        const bool both = np >= kTile && nl >= kTile;
         const bool overlap = np % kTile != 0 || nl % kTile != 0;
         const bool in_place = (addend && addend == y) || (mult && mult == y);
-        if (!(in_place && overlap) && np >= kTile && nl >= kTile && np + kTile <= lim && nl + 4 * kTile <= lim &&
-            c.x_stride[last] > 0 && (uint64_t)c.x_stride[last] <= lim && v.offset <= lim &&
-            plan.y_stride[p] <= lim && c.a_stride[last] <= 1 && c.m_stride[last] <= 1) {
-            plan.tiles_p = (uint32_t)((np + kTile - 1) / kTile);
-            const uint64_t all_tiles = plan.batches * plan.tiles_p * ((nl + kTile - 1) / kTile);
-            // whole aligned vectors in every x row, batch offset and output row
-            constexpr uint64_t E = Vec16<S>::N;
-            bool guarded = sizeof(S) == 2 && !addend && !mult && np % E == 0 && nl % E == 0 &&
-                           v.offset % E == 0 && aligned16(x) && aligned16(y);
-            for (int d = 0; d <= last; ++d)
-                if (d != p && c.x_stride[d] % (int64_t)E != 0) guarded = false;
-            const uint32_t per = guarded ? 4 : sizeof(S) == 2 && all_tiles >= 2048 && nl > kTile ? 2 : 1;
+        // whole aligned vectors in every x row, batch offset and output row
+        constexpr uint64_t E = Vec16<S>::N;
+        constexpr uint32_t kGuardedTiles = sizeof(S) == 2 ? 4 : 1;
+        bool whole = !addend && !mult && np % E == 0 && nl % E == 0 && v.offset % E == 0 && aligned16(x) &&
+                     aligned16(y);
+        for (int d = 0; d <= last; ++d)
+            if (d != p && c.x_stride[d] % (int64_t)E != 0) whole = false;
+        // With a dim below 64 the bounds-tested form, where a block still moves
+        // enough: views that one tile holds from 400 elements (us at 6.3 M
+        // elements in batches, here / adaptive tiles / one element per lane: f16
+        // 32 x 32 11.9 / 13.1 / 25, 48 x 48 8.7 / 14.1 / 25, f32 20 x 20 21.7 /
+        // 26.6 / 24.5; f32 from 256, 16 x 16 26.7 / 39 / 25.4), longer ones from 1280
+        // per block (f16 32 x 1000 10.0 / 12.3 / 26, 512 x 16 12.5 / 11.0 / 26, 504 x 8
+        // 26 / 12 / 25; f32 1000 x 32 11.3 / 12.3 / 25.5, 500 x 4 29 / 16 / 25), f32 with
+        // a short p from 2560 (40 x 1000 13.4 / 14.1 / 36, 32 x 1000 13.9 / 12.5 / 34). With
+        // both dims of 64 f32 takes it where more than one tile in 16 would
+        // overlap another one (overlapping / here, us: 12580 x 500 14.1 / 12.2,
+        // 92000 x 68 15.8 / 11.3; but 4096 x 4000 20.1 / 22.7, 3000 x 3000 16.5 /
+        // 17.1), and from 1025 to 2048 tiles, the second half of the one round
+        // that the CUs hold of either form: it wins at every shape measured there
+        // (2000 x 2560 8.3 / 7.1, 512 x 12288 9.1 / 8.1, 2688 x 2688 10.5 / 9.3; 1024
+        // tiles 5.3 / 5.5, 2500 14.3 / 15.2).
+        const uint64_t moved = std::min<uint64_t>(np, kTile) * std::min<uint64_t>(nl, kTile * kGuardedTiles);
+        const uint64_t tiles_p = (np + kTile - 1) / kTile, tiles_l = (nl + kTile - 1) / kTile;
+        const bool ragged = 16 * ((np % kTile != 0) * tiles_l + (nl % kTile != 0) * tiles_p) > tiles_p * tiles_l;
+        const uint64_t all_tiles = plan.batches * tiles_p * tiles_l;
+        const bool half_round = all_tiles > 1024 && all_tiles <= 2048;
+        constexpr bool f16 = sizeof(S) == 2;
+        const bool one_tile = np <= kTile && nl <= kTile && np * nl >= (f16 ? 400 : 256);
+        const bool guarded = whole && (both ? f16 || ragged || half_round
+                                            : one_tile || moved >= (!f16 && np < kTile ? 2560 : 1280));
+        if (fits32 && (guarded || (both && !(in_place && overlap) && c.a_stride[last] <= 1 && c.m_stride[last] <= 1))) {
+            plan.tiles_p = (uint32_t)tiles_p;
+            const uint32_t per = guarded ? kGuardedTiles : sizeof(S) == 2 && all_tiles >= 2048 && nl > kTile ? 2 : 1;
             const uint32_t spans_l = (uint32_t)((nl + per * kTile - 1) / (per * kTile));
             const uint64_t vblocks = plan.batches * plan.tiles_p * spans_l;
             if (vblocks < (uint64_t{1} << 24)) {
@@ -736,8 +763,7 @@ hipError_t launch_view(const S *x, const k::ViewArgs &v, const S *addend,
             if (per == 2) return go(view_tile_vec_kernel<S, 2, A, M>);                           \
         return go(view_tile_vec_kernel<S, 1, A, M>);                                             \
     } while (0)
-                if constexpr (sizeof(S) == 2)
-                    if (guarded) return go(view_tile_vec_kernel<S, 4, kNone, kNone, true>);
+                if (guarded) return go(view_tile_vec_kernel<S, kGuardedTiles, kNone, kNone, true>);
                 switch (ka * 3 + km) {
                     case 0: ICSDK_TILE_VEC(kNone, kNone);
                     case 1: ICSDK_TILE_VEC(kNone, kVector);
@@ -752,20 +778,32 @@ hipError_t launch_view(const S *x, const k::ViewArgs &v, const S *addend,
 #undef ICSDK_TILE_VEC
             }
         }
-        // adaptive tiles: the shorter dim whole up to 64 (32 for small
-        // tiles), the other one as long as fits the tile; views of fewer than
-        // 1024 large tiles take small ones (more, shorter blocks)
-        const bool small = n <= 1024ull * kTileElems;
-        const uint64_t elems = small ? kTileElemsSmall : kTileElems, side = small ? 32 : 64;
-        uint64_t ep = std::min(np, side), el = std::min(nl, side);
-        if (np <= nl) el = std::min(nl, std::max<uint64_t>(elems / ep / side, 1) * side);
-        else ep = std::min(np, std::max<uint64_t>(elems / el / side, 1) * side);
+        // Adaptive tiles: the shorter dim whole up to 64 (32 for small tiles),
+        // the other one as long as fits the tile. Small ones where that makes
+        // more, shorter blocks (views of fewer than 1024 large tiles), and where
+        // the large ones are mostly empty: up to twice as many small ones cost less
+        // (us, f16 at 6.3 M elements, large / small: 24 x 24, one tile either way, 36 /
+        // 20, 4 x 500 15.5 / 13.5, 8 x 500 11.8 / 13.5). A block is paid whether
+        // its tile is full or not (1.5 to 2.5 ns of the launch): tiles of fewer than
+        // 512 elements go to one element per lane, 4 ns per 1000 elements (us,
+        // here / there: 2 x 3 1530 / 25, 16 x 16 39 / 25, 16 x 32 21 / 25; with
+        // operands 2137 / 28, 55 / 28, 30 / 29).
+        uint64_t ep = 0, el = 0;
+        auto cut = [&](uint64_t elems, uint64_t side) {
+            ep = std::min(np, side), el = std::min(nl, side);
+            if (np <= nl) el = std::min(nl, std::max<uint64_t>(elems / ep / side, 1) * side);
+            else ep = std::min(np, std::max<uint64_t>(elems / el / side, 1) * side);
+            return plan.batches * ((np + ep - 1) / ep) * ((nl + el - 1) / el);
+        };
+        const uint64_t large_blocks = cut(kTileElems, 64), small_blocks = cut(kTileElemsSmall, 32);
+        const bool small = n <= 1024ull * kTileElems || small_blocks <= 2 * large_blocks;
+        const uint64_t elems = small ? kTileElemsSmall : kTileElems;
+        const uint64_t blocks = cut(elems, small ? 32 : 64);
         plan.tile_p = make_fast_div((uint32_t)ep);
         plan.tile_l = make_fast_div((uint32_t)el);
         plan.tiles_p = (uint32_t)((np + ep - 1) / ep);
         plan.tiles_l = (uint32_t)((nl + el - 1) / el);
-        const uint64_t blocks = plan.batches * plan.tiles_p * plan.tiles_l;
-        if (blocks < (uint64_t{1} << 24) && ep * el <= elems && (ep | 1u) * el <= elems / 2 * 3) {
+        if (blocks < (uint64_t{1} << 24) && (n / blocks >= 480 || blocks <= 1024) && ep * el <= elems && (ep | 1u) * el <= elems / 2 * 3) {
             auto go = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, x, addend, mult, y, plan);
                 return hipGetLastError();

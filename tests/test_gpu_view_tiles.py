@@ -84,3 +84,15 @@ def test_output_is_an_operand(sdk, orc, shape, dtype, add, mul):
     if mul:
         want = want * y.astype(np.float32)
     assert np.array_equal(ty.download(), want.astype(np_type))
+
+
+# many small transposes (more than 4 M elements: large tiles where they fill):
+# one element per lane, whole vectors in part of a tile, small and large tiles
+@pytest.mark.parametrize("shape", [(1100000, 2, 2), (700001, 2, 3), (130000, 5, 7), (65537, 8, 8), (17000, 16, 16),
+                                   (11000, 20, 20), (7400, 24, 24), (4100, 31, 33), (4200, 32, 32),
+                                   (3900, 33, 33), (2700, 40, 40), (2200, 4, 500), (2200, 500, 4), (1100, 504, 8),
+                                   (1100, 8, 504), (300, 24, 1000), (300, 1000, 24), (70, 1000, 63)])
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("add,mul", [(None, None), ("full", "second"), (None, "last")])
+def test_batched_small_transposes(sdk, orc, shape, dtype, add, mul):
+    test_transposing_view(sdk, orc, shape, (0, 2, 1), dtype, add, mul)
