@@ -11,8 +11,9 @@
 // rows]) and A = the weight: column-major [inner x cols] transposed for
 // linear (w[cols][inner] row-major), [cols x inner] as is for matmul.
 //
-// One plan (descriptors + the heuristic's first algorithm) is cached per
-// (kind, dtype, shape, bias); calls run under one mutex because the bias
+// One plan (descriptors + the heuristic's algorithms, of which the first that
+// runs is used: the library proposes some that it then refuses to launch, f16
+// 200 x 4096 -> 8192 for one) is cached per (kind, dtype, shape, bias); calls run under one mutex because the bias
 // pointer is an attribute of the cached descriptor.
 #include "gemm.hpp"
 #include "kernels.hpp"
@@ -24,6 +25,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <vector>
 
 namespace icsdk {
 namespace {
@@ -33,8 +35,11 @@ constexpr size_t kWorkspaceBytes = 32u << 20;
 struct Plan {
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t a = nullptr, b = nullptr, d = nullptr;
-    hipblasLtMatmulAlgo_t algo{};
-    size_t workspace = 0;
+    struct Algorithm {
+        hipblasLtMatmulAlgo_t algo;
+        size_t workspace;
+    };
+    std::vector<Algorithm> algorithms;   // in the heuristic's order; those that failed are taken out
 };
 
 using PlanKey = std::tuple<int, int, uint64_t, uint64_t, uint64_t, bool>;
@@ -121,11 +126,10 @@ bool make_plan(hipblasLtHandle_t handle, GemmKind kind, hipDataType type, uint64
     if (pref) hipblasLtMatmulPreferenceDestroy(pref);
     for (int i = 0; s == HIPBLAS_STATUS_SUCCESS && i < found; ++i) {
         if (results[i].state == HIPBLAS_STATUS_SUCCESS && results[i].workspaceSize <= limit) {
-            plan->algo = results[i].algo;
-            plan->workspace = results[i].workspaceSize;
-            return true;
+            plan->algorithms.push_back({results[i].algo, results[i].workspaceSize});
         }
     }
+    if (!plan->algorithms.empty()) return true;
     set_error(error, capacity, "no GEMM kernel for %llu x %llu x %llu: %s",
               (unsigned long long)m, (unsigned long long)n, (unsigned long long)k,
               s == HIPBLAS_STATUS_SUCCESS ? "none returned" : status_text(s));
@@ -182,19 +186,24 @@ bool gemm(GemmKind kind, TensorDType dtype, const void *x, const void *w, const 
             return false;
         }
     }
-    ScratchBlock workspace(plan.workspace);
-    if (plan.workspace != 0 && workspace.get() == nullptr) {
-        set_error(error, capacity, "out of device memory for the GEMM workspace");
-        return false;
-    }
     const float alpha = 1.0f, beta = 0.0f;
-    const hipblasStatus_t s = hipblasLtMatmul(g.handle, plan.desc, &alpha, w, plan.a, x, plan.b,
-                                              &beta, y, plan.d, y, plan.d, &plan.algo,
-                                              plan.workspace ? workspace.get() : nullptr,
-                                              plan.workspace, stream);
-    if (s != HIPBLAS_STATUS_SUCCESS) {
-        set_error(error, capacity, "GEMM launch failed: %s", status_text(s));
-        return false;
+    for (;;) {
+        Plan::Algorithm &use = plan.algorithms.front();
+        ScratchBlock workspace(use.workspace);
+        if (use.workspace != 0 && workspace.get() == nullptr) {
+            set_error(error, capacity, "out of device memory for the GEMM workspace");
+            return false;
+        }
+        const hipblasStatus_t s = hipblasLtMatmul(g.handle, plan.desc, &alpha, w, plan.a, x, plan.b, &beta, y,
+                                                  plan.d, y, plan.d, &use.algo, workspace.get(), use.workspace,
+                                                  stream);
+        if (s == HIPBLAS_STATUS_SUCCESS) break;
+        forget_error();
+        if (plan.algorithms.size() == 1) {
+            set_error(error, capacity, "GEMM launch failed: %s", status_text(s));
+            return false;
+        }
+        plan.algorithms.erase(plan.algorithms.begin());
     }
     return true;
 }

@@ -471,3 +471,18 @@ def test_quantized_slots(sdk, orc, fmt):
     # the scalar kernel runs the reference's chain operation for operation
     assert_bits_equal(ty2.download(), want, "device slot, unaligned: the reference's chain")
     assert dev(tx.device_ptr(), tw.device_ptr(), ty.device_ptr(), 0, inw, out) == 0
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("rows", [200, 250])
+def test_linear_where_the_first_algorithm_does_not_launch(sdk, orc, dtype, rows):
+    """4096 -> 8192 of 200 f16 rows: the GEMM library's first proposal fails at
+    its launch, the next one runs; the calls after it too."""
+    x = orc.normal((rows, 4096), 79, 0, 0.0, 1.0, dtype)
+    w = orc.normal((8192, 4096), 79, 1, 0.0, 0.05, dtype)
+    tx, tw, ty = sdk.from_numpy(x), sdk.from_numpy(w), sdk.tensor(dtype, (rows, 8192))
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    weight = abs_weight(x, w)
+    for _ in range(2):
+        sdk.call(f"tensor_linear_{dtype}", tx, tw, None, ty)
+        check(ty.download(), want.astype(x.dtype), weight, dtype, f"linear {rows}")
