@@ -121,15 +121,17 @@ __global__ __launch_bounds__(kBlock) void gemv_kernel(const T *__restrict__ x, c
 }
 
 // Small products of more input rows (and rows no GEMV can read in whole
-// vectors): each weight is used by more rows than v_dot2 carries for free, so the products go to MFMA. A block takes
-// 16 OT output columns of 16 RG input rows; its NW waves share the k range, in
-// interleaved runs of UN 128-byte lines per row, and their partial sums meet in LDS. The register layout of an MFMA operand has 16 rows in 16 neighbouring
-// lanes: loaded so from memory, every quarter of a load instruction touches 16
-// lines (16 x 8192 -> 8192 f16 42 us). So 8 lanes read a row's line, the wave
-// passes it through its own piece of LDS (16-byte vectors, the vector number
-// xor-ed with the row: conflict-free both ways), and the next run's loads are
-// in flight meanwhile. Lane (i, g) of the MFMA takes vector 4 c + g of row i
-// as chunk c: the k order inside a chunk is the memory's, the same for both.
+// vectors): each weight is used by more rows than v_dot2 carries for free, so
+// the products go to MFMA. A block takes 16 OT output columns of 16 RG input
+// rows; its NW waves share the k range, in interleaved runs of UN 128-byte lines
+// per row, and their partial sums meet in LDS. The register layout of an MFMA
+// operand has 16 rows in 16 neighbouring lanes: loaded so from memory, every
+// quarter of a load instruction touches 16 lines (16 x 8192 -> 8192 f16 42 us).
+// So 8 lanes read a row's line, the wave passes it through its own piece of LDS
+// (16-byte vectors, the vector number xor-ed with the row: conflict-free both
+// ways), and the next run's loads are in flight meanwhile. Lane (i, g) of the
+// MFMA takes vector 4 c + g of row i as chunk c: the k order inside a chunk is
+// the memory's, the same for both.
 // Bound: a block's operands through its CU (x again for every 16 columns),
 // a few memory latencies in a row, and the launch.
 template <typename T, int RG, int OT, int NW, int UN>
@@ -293,23 +295,26 @@ hipError_t launch_skinny(const T *x, const T *w, const T *bias, T *y, size_t row
 }
 
 // Small products on skinny_kernel, or hipErrorNotSupported. The library's call
-// takes 10.6 us or more at any size (rows that are no whole number of 16-byte
-// vectors up to 48) and streams large weights better. us here, library's in
-// brackets:
+// takes 7.1 us or more at any size, one call after another, and streams large
+// weights better. us per call here, the library's in brackets, calls in a row
+// with other buffers each time (a call that is waited for gains more: 16 x 4096
+// -> 4096 21.0 [24.5], 128 x 2048 -> 1000 17.8 [21.6]):
 //   up to 32 input rows: f16 weights of rows of up to 8 KB, 34 MB in all (16 x
-//   4096 -> 4096 9.5 [10.9], 32 x 4096 -> 4096 10.6 [11.4], 16 x 2048 -> 2048 4.5
-//   [11.1]; but 16 x 8192 -> 2048 12.3 [11.2], 32 x 4096 -> 14336 28 [25]), or of 12
-//   KB and 13 MB (16 x 6144 -> 1000 6.9 [11.3]); f32, whose MFMAs are 16 times
-//   slower, of 16 KB and 17 MB (16 x 2048 -> 2048 6.9 [10.9], 32 x 4096 -> 1024 10.0
-//   [11.3]; but 16 x 6144 -> 1000 14.5 [13.7]);
-//   up to 64: rows of 8 KB, f16 13 MB, f32 17 MB (64 x 4096 -> 1024 f16 6.8 [10.9],
-//   f32 16 [11.5]);
-//   above: 64 rows per block; f16 where 16-column blocks fit one round of the
-//   256 CUs (128 x 4096 -> 1024 9.9 [12.6]), or 32-column blocks are no more than
-//   512 and read up to 1 M bytes of k together (400 x 752 -> 1536 8.7 [11.1], 1000
-//   x 776 -> 668 9.3 [11.9]; but 400 x 1848 -> 1944 18 [15.5], 1000 x 360 -> 2318 14.4
-//   [12.7]); f32 where 16-column blocks fit and rows are up to 4 KB (200 x 776
-//   -> 668 8.8 [11.5]; but 400 x 776 -> 668 13.7 [12.4]).
+//   4096 -> 4096 8.7 [10.2], 32 x 4096 -> 4096 9.9 [12.7], 16 x 2048 -> 2048 4.9
+//   [8.3]), or of 12 KB and 13 MB (16 x 6144 -> 1000 6.4 [10.9]); f32, whose MFMAs
+//   are 16 times slower, of 16 KB and 17 MB (16 x 2048 -> 2048 6.5 [9.1], 32 x 4096
+//   -> 1024 9.8 [12.7]);
+//   up to 64: rows of 8 KB, 13 MB in all (64 x 4096 -> 1024 f16 5.4 [8.6], f32 64 x
+//   1536 -> 2048 7.6 [8.3]; but f32 64 x 1024 -> 4096 9.9 [9.4]);
+//   above: 64 rows per block; 16-column blocks where they fit one round of the
+//   256 CUs, f16 to rows of 4 KB (128 x 2048 -> 1000 6.3 [7.4], 100 x 2048 -> 64 5.5
+//   [7.3]; but 100 x 3072 -> 200 7.8 [7.3], 128 x 4096 -> 512 9.0 [7.5]), beyond 512
+//   input rows of 3 KB (1000 x 1536 -> 200 7.1 [7.2]; but 1000 x 2048 -> 200 8.3
+//   [7.6]), f32 of 2.5 KB (200 x 576 -> 1000 6.9 [7.5]; but 256 x 770 -> 200 8.5 [7.1]);
+//   f16 32-column blocks that are no more than 256 and read up to 1 M bytes of k
+//   together (512 x 2048 -> 1000 8.2 [9.1], 400 x 752 -> 1536 8.0 [8.4]), or no more
+//   than 512 with rows of 1.25 KB (1000 x 576 -> 1000 6.8 [7.5]; but 200 x 1024 ->
+//   4096 8.9 [8.2], 512 x 770 -> 2048 8.8 [8.4]).
 template <typename T>
 hipError_t skinny(const T *x, const T *w, const T *bias, T *y, size_t rows, size_t in, size_t out,
                   hipStream_t s) {
@@ -320,15 +325,15 @@ hipError_t skinny(const T *x, const T *w, const T *bias, T *y, size_t rows, size
     if (rows > 64) {
         if (rows > (size_t{1} << 20)) return hipErrorNotSupported;
         const size_t narrow = tiles * ((rows + 63) / 64), wide = (tiles + 1) / 2 * ((rows + 63) / 64);
-        if (narrow <= 256 && row <= (f32 ? 4096u : 8192u))
+        if (narrow <= 256 && row <= (f32 ? 2560u : rows <= 512 ? 4096u : 3072u))
             return launch_skinny<T, 4, 1, 8, 1>(x, w, bias, y, rows, in, out, s);
         if constexpr (!f32)
-            if (wide <= 512 && row <= 4096 && wide * row <= (1u << 20))
+            if (row <= (rows <= 512 ? 4096u : 3072u) && (wide <= 256 ? wide * row <= (1u << 20) : wide <= 512 && row <= 1280))
                 return launch_skinny<T, 4, 2, 4, 1>(x, w, bias, y, rows, in, out, s);
         return hipErrorNotSupported;
     }
     const bool few = rows <= 32;
-    const bool small = f32 ? total <= (17u << 20) && row <= (few ? 16384u : 8192u)
+    const bool small = f32 ? (few ? total <= (17u << 20) && row <= 16384u : total <= (13u << 20) && row <= 8192u)
                            : (total <= (34u << 20) && row <= 8192u && few) ||
                                  (total <= (13u << 20) && row <= (few ? 12288u : 8192u));
     if (!small) return hipErrorNotSupported;
