@@ -1010,12 +1010,17 @@ __global__ __launch_bounds__(BM * 2 * KS) void sdpa_flash_f32_kernel(const float
         const uint32_t t = t0 + kpart;
         const uint32_t k0 = t * KN;
         const bool more = t0 + KS < tiles;
-        // the mask of the wave's scores, asked for before the next step's tiles
-        // (see the f16 kernel; 32q/8kv 2048 x 2048 D 64 500 -> 349 us)
+        // The mask of the wave's scores, asked for before the next step's tiles
+        // (see the f16 kernel; 32q/8kv 2048 x 2048 D 64 500 -> 349 us). Unlike
+        // there the last step has its branch: without it the D 128 form spilled 8
+        // registers, and short key ranges fetched a tile more (us, without ->
+        // with: 32q/8kv 2048 x 2048 670 -> 602, 8 x 32q/8kv 16 x 2048 323 -> 169, 512
+        // x 4 heads 49 x 49 124 -> 95).
         f32x4 mq[kMask ? 4 : 1];
         if constexpr (kMask) {
             const float *mrow = mask + (size_t)(q_live ? qi : 0) * a.kl;
-            if (k0 + KN <= a.kl) {
+            if (!wave_live) {   // (dead waves of a last block only move tiles)
+            } else if (k0 + KN <= a.kl) {
 #pragma unroll
                 for (int g = 0; g < 4; ++g) mq[g] = *reinterpret_cast<const f32x4_4 *>(mrow + k0 + 8 * g + 4 * half);
             } else {
@@ -1025,7 +1030,7 @@ __global__ __launch_bounds__(BM * 2 * KS) void sdpa_flash_f32_kernel(const float
                     for (int i = 0; i < 4; ++i) mq[g][i] = mrow[min(k0 + 8 * g + 4 * half + i, a.kl - 1)];
             }
         }
-        if (kMask || more) fetch((t0 + KS) * KN);
+        if (more) fetch((t0 + KS) * KN);
         const float *kt = &lds[buf * 2 * KS * TILE + kpart * TILE];   // this wave's K tile
         const float *vt = kt + KS * TILE;                              // and V tile
         if (t < tiles && wave_live && !(a.causal && (uint64_t)k0 > wave_last_key)) {

@@ -482,7 +482,11 @@ hipError_t fold(const DecodePlan &p, const S *q, const S *k, const S *v, const S
 // mostly idle either way. Measured (us, flash -> here): 4 x 32q/8kv 8 x 2048
 // D 128 f16 22.8 -> 18.5, 2 x 32q/4kv 8 x 4096 23.7 -> 17.0, f32 4 x 32q/8kv 16
 // x 2048 87 -> 50, 12 x 24 x 2048 47.5 -> 19.3; excluded, f16 4 x 32q/8kv 16
-// x 2048 23.3 vs 27.3, 8 x 12 x 24 x 600 14.1 vs 22.5, f32 35.0 vs 36.3.
+// x 2048 23.3 vs 27.3, 8 x 12 x 24 x 600 14.1 vs 22.5, f32 35.0 vs 36.3. Where no
+// heads share a kv head, f16 calls of dims 64 and 128 over long ranges are a
+// little faster there (4 x 8 heads 16 x 2048 D 128 13.1 vs 15.6, 64 x 8 heads 1 x
+// 2048 D 64 41.5 vs 44.7); they stay here for their P, an f16 pair instead of one f16
+// (relative error of the outputs 2.0e-4, there 2.9e-4).
 DecodePlan decode_plan(const k::SdpaShape &sh, bool aligned, bool f32, bool causal) {
     DecodePlan p;
     const size_t e = f32 ? 4 : 8, wide = sh.head_dim > sh.value_dim ? sh.head_dim : sh.value_dim;
