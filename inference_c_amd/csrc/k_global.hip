@@ -374,15 +374,16 @@ hipError_t no_alloc_scratch(void **ptr) {
     return hipSuccess;
 }
 
-// Pass-1 chunk for nvec vectors: the smallest whose blocks still number at
-// most 1024 (32 KiB chunks up to 32 MiB, 128 KiB up to 128 MiB), else 1 MiB.
-// Small tensors need many short blocks to fill the chip, large ones few long
-// ones (us per call, 1 MiB chunks everywhere -> here: 1000 f32 12.1 -> 4.0
-// (one block), 2^20 20.1 -> 6.4, 2^22 26.9 -> 6.3, 2^23 27.3 -> 7.0, 2^25 29.6
-// -> 22.2; 2^26 41.7 with 1 MiB, 42.0 with 128 KiB).
+// Pass-1 chunk for nvec vectors: 32 KiB up to 1024 blocks (32 MiB), 128 KiB until
+// 1 MiB chunks give every CU a block (256 MiB). Small tensors need many short
+// blocks to fill the chip, large ones few long ones (us per call in a row on
+// one tensor, 1 MiB chunks everywhere -> here: 1000 f32 12.5 -> 3.8 (one block),
+// 2^20 20.5 -> 7.2, 2^22 25.4 -> 7.2 (another tensor each time 8.0), 2^24 28.4 ->
+// 13.8, 2^25 + 4 29.0 -> 22.5, 2^26 - 4 44.0 -> 42.1; 3 x 2^24 the same; at 2^26
+// 128 KiB chunks 42.0, 1 MiB 41.6).
 static size_t sum_max_chunk_for(size_t nvec) {
     if (nvec <= kChunkSmall * 1024) return kChunkSmall;
-    if (nvec <= kChunkMid * 1024) return kChunkMid;
+    if (nvec < kChunkLarge * 256) return kChunkMid;
     return kChunkLarge;
 }
 

@@ -44,3 +44,15 @@ def test_argmax_sizes(sdk, orc, dtype, vec, n_of):
     tx.upload(x)
     sdk.call(f"tensor_argmax_{dtype}", tx, ti)
     assert ti.download()[0] == 0
+
+
+@pytest.mark.parametrize("n", [(1 << 26) - 4, (1 << 26) + 3])
+def test_sum_max_around_the_largest_chunk(sdk, orc, n):
+    """2048 chunks of 128 KiB (two partials per folding lane), 256 of 1 MiB."""
+    x = orc.uniform((n,), 47, 0, -1.0, 1.0)
+    x[n - 1], x[n // 3] = 2.5, 3.5
+    ts, tm = sdk.tensor("f64", (1,)), sdk.tensor("f32", (1,))
+    sdk.call("tensor_sum_max_f32", sdk.from_numpy(x), ts, tm)
+    want_s, abs_s, want_m = orc.sum_max(x)
+    assert abs(float(ts.download()[0]) - want_s) <= 32 * 2.0 ** -24 * abs_s
+    assert tm.download()[0] == want_m
