@@ -143,3 +143,64 @@ def test_softmax_in_place_cut_rows(sdk, orc):
         sdk.call("tensor_softmax_f32", tx, 0, tx)
         want = softmax64(x, False, 2)
         assert (np.abs(tx.download() - want) <= 1e-5 * want).all()
+
+
+# rows cut into parts: whole last vectors, ragged ones that overlap the one
+# before, a last part that joined the one before it
+@pytest.mark.parametrize("rows,width", [(2, 65536), (3, 65531), (2, 2047 * 8 * 5 + 1)])
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_cut_rows_in_place(sdk, orc, rows, width, dtype):
+    """y over x: every load of a part comes before any store of it."""
+    x = orc.normal((rows, width), 87, 0, 0.3, 1.0, dtype)
+    w = orc.uniform((width,), 87, 1, 0.5, 1.5, dtype)
+    b = orc.uniform((width,), 87, 2, -0.5, 0.5, dtype)
+    tw, tb = sdk.from_numpy(w), sdk.from_numpy(b)
+    d = x.astype(np.float64)
+    c = d - d.mean(-1, keepdims=True)
+    soft = softmax64(x, False, rows)
+    for name, args, want in (
+            ("rms_norm", (tw, 1e-6), d / np.sqrt((d * d).mean(-1, keepdims=True) + 1e-6) * w),
+            ("layer_norm", (tw, tb, 1e-5), c / np.sqrt((c * c).mean(-1, keepdims=True) + 1e-5) * w + b),
+            ("softmax", (0,), soft)):
+        tx = sdk.from_numpy(x)
+        sdk.call(f"tensor_{name}_{dtype}", tx, *args, tx)
+        got = tx.download().astype(np.float64)
+        # as in the tests above: the output's rounding, the sums' in f32
+        tol = 2.0 ** -10 if dtype == "f16" else 1e-5
+        floor = (2.0 ** -24 if dtype == "f16" else 1e-30) if name == "softmax" else tol
+        assert (np.abs(got - want) <= tol * np.abs(want) + floor).all(), name
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_captured_long_rows(sdk, orc, dtype):
+    """Rows that an eager call cuts, with partial results in scratch memory,
+    are recorded as one kernel without; replays give what the eager call does
+    up to the sums' order."""
+    import ctypes
+    hip = sdk.lib
+    hip.tensor_device_hip_stream.restype = ctypes.c_void_p
+    stream = ctypes.c_void_p(hip.tensor_device_hip_stream())
+    x = orc.normal((2, 65531), 88, 0, 0.0, 2.0, dtype)
+    tx, ty = sdk.from_numpy(x), sdk.tensor(dtype, x.shape)
+    call = (f"tensor_softmax_{dtype}", tx, 0, ty)
+    want = softmax64(x, False, 2)
+    tol = 2.0 ** -10 * want + 2.0 ** -24 if dtype == "f16" else 1e-5 * want + 1e-30
+    graph, exe, nodes = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t()
+    sdk.call(*call)
+    ty.download()
+    assert hip.hipStreamBeginCapture(stream, 2) == 0     # relaxed
+    try:
+        sdk.call(*call)
+    finally:
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+    assert nodes.value == 1
+    assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        ty.upload(np.zeros_like(x))
+        assert hip.hipGraphLaunch(exe, stream) == 0
+        assert (np.abs(ty.download() - want) <= tol).all()
+        sdk.call(*call)          # eager work between the replays
+        assert (np.abs(ty.download() - want) <= tol).all()
+    assert hip.hipGraphExecDestroy(exe) == 0
+    assert hip.hipGraphDestroy(graph) == 0
