@@ -13,8 +13,9 @@
 //
 // One plan (descriptors + the heuristic's algorithms, of which the first that
 // runs is used: the library proposes some that it then refuses to launch, f16
-// 200 x 4096 -> 8192 for one) is cached per (kind, dtype, shape, bias); calls run under one mutex because the bias
-// pointer is an attribute of the cached descriptor.
+// 200 x 4096 -> 8192 for one) is cached per (kind, dtype, shape, bias); calls
+// run under one mutex because the bias pointer is an attribute of the cached
+// descriptor.
 #include "gemm.hpp"
 #include "kernels.hpp"
 

@@ -552,8 +552,6 @@ hipError_t sdpa_f16(const uint16_t *q, const uint16_t *k, const uint16_t *v,
 #undef ICSDK_FLASH_SHAPES_F16
 #undef ICSDK_FLASH_SHAPES_F32
 #undef ICSDK_FLASH_VARIANTS_KS2_BM
-#undef ICSDK_FLASH_VARIANTS_KS2
 #undef ICSDK_FLASH_VARIANTS_KS
-
 
 }  // namespace icsdk

@@ -3,15 +3,15 @@
 // K and V are read once per kv head, and the key range is spread over waves
 // and blocks.
 //
-// The rows of a kv head -- its `group` query heads times q_len positions --
-// are consecutive in q and out, so packed row r is row r of a [group * q_len,
-// D] matrix; its position is r % q_len. A wave holds 16 rows (more rows: more
+// The rows of a kv head -- its `group` query heads times q_len positions -- are
+// consecutive in q and out, so packed row r is row r of a [group * q_len, D]
+// matrix; its position is r % q_len. A wave holds 16 rows (more rows: more
 // blocks, which read K and V from the caches; 32 or 64 rows per wave measured
-// slower, one wave per SIMD) and walks key tiles of 32 (f16) or 16 (f32) keys; a block's four waves take
-// every fourth tile of the block's part of the keys, with nothing shared
-// until the end: K and V go from memory straight into the MFMA operands'
-// registers, the next tile's loads issued before the current tile is
-// computed. No LDS, no barrier in the loop.
+// slower, one wave per SIMD) and walks key tiles of 32 (f16) or 16 (f32) keys;
+// a block's four waves take every fourth tile of the block's part of the keys,
+// with nothing shared until the end: K and V go from memory straight into the
+// MFMA operands' registers, the next tile's loads issued before the current
+// tile is computed. No LDS, no barrier in the loop.
 //
 // v_mfma_f32_16x16x32_f16 (f16) and 16x16x4_f32: A[m][k] in lane l at m = l %
 // 16, k = 8 g + i (f32: k = g), g = l / 16; B[k][n] at n = l % 16 likewise;

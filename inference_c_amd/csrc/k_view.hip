@@ -413,24 +413,24 @@ __global__ __launch_bounds__(kBlock) void view_tile_kernel(const S *__restrict__
 // 64 x 64 tiles in 16-byte vectors of E elements (8 for f16, 4 for f32), for
 // views whose p and last dimensions have at least 64 elements: a tile's 64 x
 // rows (64 elements along p, contiguous in x) are read as 64 / E vectors each
-// into LDS rows [l], vector c of row l at slot c ^ (l / E); each output row
-// (64 elements along the last dim, contiguous in y) is gathered from one LDS
+// into LDS rows [l], vector c of row l at slot c ^ (l / E); each output row (64
+// elements along the last dim, contiguous in y) is gathered from one LDS
 // column, E reads per vector, and written as 64 / E vectors. With the slot
-// swizzle the 64 lanes of a gather read distinct banks (f16: 32, lanes 2m
-// and 2m + 1 sharing a dword; f32: 64). A last tile that would reach past the
-// end starts 64 elements before it instead and writes the overlap with the
-// same values, so no access needs a bounds test; vectors are loaded and
-// stored at any element alignment. A block takes kTiles tiles along the last dim: two for f16 where
-// that still leaves 1024 blocks, else one (f16 with an addend, one / two /
-// four tiles: [3000, 3000] 13.7 / 10.0 / 11.3 us, [8192, 8192] 48.9 / 47.0 /
-// 47.9, [4096, 4096] 13.4 / 15.0 / 16.4). kGuarded: the form for whole
+// swizzle the 64 lanes of a gather read distinct banks (f16: 32, lanes 2m and
+// 2m + 1 sharing a dword; f32: 64). A last tile that would reach past the end
+// starts 64 elements before it instead and writes the overlap with the same
+// values, so no access needs a bounds test; vectors are loaded and stored at
+// any element alignment. A block takes kTiles tiles along the last dim: two for
+// f16 where that still leaves 1024 blocks, else one (f16 with an addend, one /
+// two / four tiles: [3000, 3000] 13.7 / 10.0 / 11.3 us, [8192, 8192] 48.9 /
+// 47.0 / 47.9, [4096, 4096] 13.4 / 15.0 / 16.4). kGuarded: the form for whole
 // aligned vectors without operands: bounds tests instead of the overlap (the
 // launcher says where), f16 with four tiles, each load waited for before the
-// next, which is the faster one there ([4096, 4000] 11.6 us against 12.7-12.8, [64, 512, 512] 12.4 against
-// 13.2-15.6). Operands enter as a vector along the last dim or as one element per
-// output row (OperandKind), loaded before the barrier. Against the
-// one-element-per-lane tiles: f16 [4097, 4095] 30.0 -> 21.4 us, [4096,
-// 4096] with both operands 41.0 -> 15.1, f32 39.6 -> 26.0.
+// next, which is the faster one there ([4096, 4000] 11.6 us against 12.7-12.8,
+// [64, 512, 512] 12.4 against 13.2-15.6). Operands enter as a vector along the
+// last dim or as one element per output row (OperandKind), loaded before the
+// barrier. Against the one-element-per-lane tiles: f16 [4097, 4095] 30.0 ->
+// 21.4 us, [4096, 4096] with both operands 41.0 -> 15.1, f32 39.6 -> 26.0.
 //
 // Everything a wave needs before its first load arrives as a plain scalar
 // argument (preloaded in SGPRs; the tile grid split by multiply-high
