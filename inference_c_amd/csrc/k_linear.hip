@@ -295,10 +295,11 @@ hipError_t launch_skinny(const T *x, const T *w, const T *bias, T *y, size_t row
 }
 
 // Small products on skinny_kernel, or hipErrorNotSupported. The library's call
-// takes 7.1 us or more at any size, one call after another, and streams large
-// weights better. us per call here, the library's in brackets, calls in a row
-// with other buffers each time (a call that is waited for gains more: 16 x 4096
-// -> 4096 21.0 [24.5], 128 x 2048 -> 1000 17.8 [21.6]):
+// is bound by its host part, 7.1 us one after another on one host and 8.4 on
+// another, and streams large weights better. us per call here, the library's
+// in brackets, calls in a row with other buffers each time on the faster host
+// (a call that is waited for gains more: 16 x 4096 -> 4096 21.0 [24.5], 128 x
+// 2048 -> 1000 17.8 [21.6], 100 x 3072 -> 200 19.0 [20.8]):
 //   up to 32 input rows: f16 weights of rows of up to 8 KB, 34 MB in all (16 x
 //   4096 -> 4096 8.7 [10.2], 32 x 4096 -> 4096 9.9 [12.7], 16 x 2048 -> 2048 4.9
 //   [8.3]), or of 12 KB and 13 MB (16 x 6144 -> 1000 6.4 [10.9]); f32, whose MFMAs
@@ -307,14 +308,16 @@ hipError_t launch_skinny(const T *x, const T *w, const T *bias, T *y, size_t row
 //   up to 64: rows of 8 KB, 13 MB in all (64 x 4096 -> 1024 f16 5.4 [8.6], f32 64 x
 //   1536 -> 2048 7.6 [8.3]; but f32 64 x 1024 -> 4096 9.9 [9.4]);
 //   above: 64 rows per block; 16-column blocks where they fit one round of the
-//   256 CUs, f16 to rows of 4 KB (128 x 2048 -> 1000 6.3 [7.4], 100 x 2048 -> 64 5.5
-//   [7.3]; but 100 x 3072 -> 200 7.8 [7.3], 128 x 4096 -> 512 9.0 [7.5]), beyond 512
-//   input rows of 3 KB (1000 x 1536 -> 200 7.1 [7.2]; but 1000 x 2048 -> 200 8.3
-//   [7.6]), f32 of 2.5 KB (200 x 576 -> 1000 6.9 [7.5]; but 256 x 770 -> 200 8.5 [7.1]);
+//   256 CUs, f16 to rows of 6 KB (128 x 2048 -> 1000 6.3 [7.4], 100 x 2048 -> 64 5.5
+//   [7.3], 100 x 3072 -> 200 7.8 [7.3]; but 128 x 4096 -> 512 9.0 [7.5]), 4 KB where
+//   they are no whole vectors (128 x 3002 -> 200 10.7 [8.7]), beyond 512 input rows
+//   of 3 KB (1000 x 1536 -> 200 7.1 [7.2]; but 1000 x 2048 -> 200 8.3 [7.6], 1000 x
+//   3072 -> 200 11.1 [9.2]), f32 of 2.5 KB (200 x 576 -> 1000 6.9 [7.5]; but 128 x 770
+//   -> 200 8.2 [7.2], 256 x 1024 -> 200 8.9 [7.2]);
 //   f16 32-column blocks that are no more than 256 and read up to 1 M bytes of k
 //   together (512 x 2048 -> 1000 8.2 [9.1], 400 x 752 -> 1536 8.0 [8.4]), or no more
-//   than 512 with rows of 1.25 KB (1000 x 576 -> 1000 6.8 [7.5]; but 200 x 1024 ->
-//   4096 8.9 [8.2], 512 x 770 -> 2048 8.8 [8.4]).
+//   than 512 with rows of 1.6 KB (1000 x 576 -> 1000 6.8 [7.5], 512 x 770 -> 2048 8.8
+//   [8.4]; but 200 x 1024 -> 4096 8.9 [8.2]).
 template <typename T>
 hipError_t skinny(const T *x, const T *w, const T *bias, T *y, size_t rows, size_t in, size_t out,
                   hipStream_t s) {
@@ -325,10 +328,10 @@ hipError_t skinny(const T *x, const T *w, const T *bias, T *y, size_t rows, size
     if (rows > 64) {
         if (rows > (size_t{1} << 20)) return hipErrorNotSupported;
         const size_t narrow = tiles * ((rows + 63) / 64), wide = (tiles + 1) / 2 * ((rows + 63) / 64);
-        if (narrow <= 256 && row <= (f32 ? 2560u : rows <= 512 ? 4096u : 3072u))
+        if (narrow <= 256 && row <= (f32 ? 2560u : rows > 512 ? 3072u : row % 16 == 0 ? 6144u : 4096u))
             return launch_skinny<T, 4, 1, 8, 1>(x, w, bias, y, rows, in, out, s);
         if constexpr (!f32)
-            if (row <= (rows <= 512 ? 4096u : 3072u) && (wide <= 256 ? wide * row <= (1u << 20) : wide <= 512 && row <= 1280))
+            if (row <= (rows <= 512 ? 4096u : 3072u) && (wide <= 256 ? wide * row <= (1u << 20) : wide <= 512 && row <= 1600))
                 return launch_skinny<T, 4, 2, 4, 1>(x, w, bias, y, rows, in, out, s);
         return hipErrorNotSupported;
     }

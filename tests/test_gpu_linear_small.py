@@ -48,8 +48,8 @@ def test_special_values_stay_in_their_rows(sdk, dtype, rows, inner, out):
 
 # either side of the limits on a row's bytes and on the blocks
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
-@pytest.mark.parametrize("rows,inner,out", [(100, 2048, 70), (100, 2050, 70), (520, 1536, 40), (520, 1537, 40),
-                                            (300, 640, 700), (300, 641, 700), (512, 2048, 500), (700, 600, 1000),
-                                            (64, 1664, 2048), (64, 1700, 2048)])
+@pytest.mark.parametrize("rows,inner,out", [(100, 3072, 70), (100, 3073, 70), (520, 1536, 40), (520, 1537, 40),
+                                            (300, 775, 700), (300, 776, 700), (512, 2048, 500), (700, 800, 1000),
+                                            (700, 801, 1000), (520, 640, 200), (64, 1664, 2048), (64, 1700, 2048)])
 def test_limits_of_the_small_kernel(sdk, orc, dtype, rows, inner, out):
     test_few_rows(sdk, orc, dtype, True, rows, inner, out)
